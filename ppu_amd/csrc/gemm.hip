@@ -74,45 +74,13 @@
 // rows and a K range (consecutive M tiles) run on one XCD and read the
 // weights into one L2: with U units and U % 8 == 0, workgroup b (XCD b % 8)
 // takes unit (b % 8) * U / 8 + b / 8, M tile fastest.
-#include "q35_common.hpp"
+#include "gemm_ksplit.hpp"
 
 namespace {
 
-enum { KIND_BF16 = 0, KIND_SWIGLU = 1, KIND_I32 = 2, KIND_DEQ = 3, KIND_DEQ_SWIGLU = 4 };
-constexpr int kNumKinds = 5;
 constexpr int kMaxSplitTiles = 8192;  // counters at the start of a split-K workspace
 constexpr int kCounterBytes = kMaxSplitTiles * 4;
 
-struct GemmArgs {
-  const uint8_t* A;  // [M, K]
-  const uint8_t* B;  // [N, K] (SwiGLU kinds: [2N, K])
-  void* C;           // [M, N] bf16 or int32
-  int M, N, K;       // K in elements
-  const float* s_x;  // int8 kinds 3, 4: per-row scales of A
-  const float* s_w;  // per-row scales of B
-  unsigned* cnt;     // split-K arrival counters, one per tile
-  uint8_t* part;     // split-K partial tiles
-  int splits, kps;   // splits per tile, stages per split
-};
-
-typedef __attribute__((address_space(3))) uint8_t lds_u8;
-Q35_DEV uint32_t lds_offset(const void* p) { return (uint32_t)(uintptr_t)(const lds_u8*)p; }
-
-// One wave instruction of the stage ring: lane i copies the 16 bytes at
-// sbase + voff to LDS bytes [lds + 16 i, +16) (the LDS base goes in m0).
-Q35_DEV void dma16(uint32_t lds, const uint8_t* sbase, uint32_t voff) {
-  asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
-}
-// s_waitcnt vmcnt(N) (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt
-// and lgkmcnt at their "no wait" maxima). As a builtin the compiler's wait
-// pass sees it and keeps it; it does not know of the asm loads it waits for.
-template <int N>
-Q35_DEV void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-// This wave's LDS reads complete (s_waitcnt lgkmcnt(0)).
-Q35_DEV void wait_lds() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (3 << 14)); }
 // Workgroup barrier; the empty asm statements keep the compiler from moving
 // memory accesses across it (the builtin barrier alone does not order them).
 Q35_DEV void ring_barrier() {
@@ -120,38 +88,12 @@ Q35_DEV void ring_barrier() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
-// Keeps the compiler's scheduler from moving any instruction across it, so
-// the MFMA / read / DMA interleave below is issued as written.
-#define Q35_PIN() __builtin_amdgcn_sched_barrier(0)
-
-typedef float q35_f32x16 __attribute__((ext_vector_type(16)));
-typedef int q35_i32x16 __attribute__((ext_vector_type(16)));
-typedef int q35_i32x4 __attribute__((ext_vector_type(4)));
-Q35_DEV q35_f32x16 mfma32(const q35_u32x4 a, const q35_u32x4 b, q35_f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(q35_bf16x8, a),
-                                                 __builtin_bit_cast(q35_bf16x8, b), c, 0, 0, 0);
-}
-Q35_DEV q35_i32x16 mfma32(const q35_u32x4 a, const q35_u32x4 b, q35_i32x16 c) {
-  return __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(q35_i32x4, a),
-                                               __builtin_bit_cast(q35_i32x4, b), c, 0, 0, 0);
-}
-template <bool I8> struct GemmAcc { using T = q35_f32x16; using E = float; };
-template <> struct GemmAcc<true> { using T = q35_i32x16; using E = int; };
 Q35_DEV uint32_t acc_bits(float v) { return __float_as_uint(v); }
 Q35_DEV uint32_t acc_bits(int v) { return (uint32_t)v; }
 Q35_DEV float acc_from(uint32_t b, float) { return __uint_as_float(b); }
 Q35_DEV int acc_from(uint32_t b, int) { return (int)b; }
 
-constexpr bool kind_i8(int kind) { return kind >= KIND_I32; }
-constexpr bool kind_swiglu(int kind) { return kind == KIND_SWIGLU || kind == KIND_DEQ_SWIGLU; }
-
 template <bool V> struct BoolTag { static constexpr bool value = V; };
-
-// Slot of 16-byte chunk c of tile row r in the swizzled LDS image.
-template <int RB>
-Q35_DEV int swz(int r) {
-  return RB == 64 ? (r >> 2) & 3 : (r >> 1) & 7;
-}
 
 template <int WM, int WN, int FM, int FN, int RB, int NSA, int NSB, bool ROT, int KIND, bool SPLIT, bool STAGED>
 __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
@@ -617,6 +559,37 @@ constexpr bool kStaged[kTiles] = {true, true, true, true, true, false, false, fa
 constexpr bool kSplitOk[kTiles] = {false, true, true, true, false, false, true, true, true};  // up to 8 blocks per wave
 constexpr int kMaxSplits = 8;
 
+// Tiles of the K-splitting kernel, by operand rows (32 FN weight rows, 16 for
+// a half tile, + 32 FM tokens): FN, FM, waves, ring pieces per wave, half tile;
+// built for the SwiGLU kinds, for the others. Rings and waves from a sweep over
+// the model's shapes at 17 to 1024 tokens.
+#define Q35_GEMM_KS_TILES(X)                \
+  X(0, 1, 1, 4, 3, true, false, true)       \
+  X(1, 1, 1, 8, 2, false, false, true)      \
+  X(2, 2, 1, 4, 3, false, true, true)       \
+  X(3, 1, 2, 4, 3, false, false, true)      \
+  X(4, 2, 2, 4, 2, false, true, true)       \
+  X(5, 1, 3, 4, 2, false, false, true)      \
+  X(6, 2, 3, 4, 1, false, true, true)       \
+  X(7, 3, 2, 4, 1, false, false, true)      \
+  X(8, 4, 2, 4, 1, false, false, true)      \
+  X(9, 2, 4, 4, 1, false, true, true)       \
+  X(10, 4, 3, 4, 1, false, true, false)     \
+  X(11, 4, 4, 4, 1, false, true, false)
+constexpr int kKsTiles = 12;
+#define Q35_GEMM_KS_W(id, fn, fm, w, s, half, sg, pl) (half) ? 16 : 32 * fn,
+#define Q35_GEMM_KS_T(id, fn, fm, w, s, half, sg, pl) 32 * fm,
+#define Q35_GEMM_KS_SG(id, fn, fm, w, s, half, sg, pl) sg,
+#define Q35_GEMM_KS_PL(id, fn, fm, w, s, half, sg, pl) pl,
+constexpr int kKsWeights[kKsTiles] = {Q35_GEMM_KS_TILES(Q35_GEMM_KS_W)};
+constexpr int kKsTokens[kKsTiles] = {Q35_GEMM_KS_TILES(Q35_GEMM_KS_T)};
+constexpr bool kKsSwiglu[kKsTiles] = {Q35_GEMM_KS_TILES(Q35_GEMM_KS_SG)};
+constexpr bool kKsPlain[kKsTiles] = {Q35_GEMM_KS_TILES(Q35_GEMM_KS_PL)};
+#undef Q35_GEMM_KS_W
+#undef Q35_GEMM_KS_T
+#undef Q35_GEMM_KS_SG
+#undef Q35_GEMM_KS_PL
+
 long long tiles_of(int tile, int M, int N, int kind) {
   const int nc = kind_swiglu(kind) ? kTN[tile] / 2 : kTN[tile];
   return (long long)((M + kTM[tile] - 1) / kTM[tile]) * ((N + nc - 1) / nc);
@@ -633,10 +606,32 @@ long long workspace_bytes(int tile, int M, int N, int kind, int splits) {
 // staged epilogue for SwiGLU and dequant; outputs with fewer tiles than CUs
 // split K only when each split keeps at least 40 stages (the partial-tile
 // exchange costs more than the idle CUs below that).
+//
+// Outputs of few tokens or few columns run on the K-splitting kernel instead
+// (tile kTiles + its index): the smallest of its tiles that covers the output
+// with one workgroup per CU, as long as the tile's operand rows stay few
+// enough. Measured at the edges (us, this kernel against the ring plans, cold
+// weights): 2048x2048 bf16 M = 33 5.4 / 13.5, 340 9.9 / 13.8, 1024 15.0 / 14.9;
+// 2048x6144 bf16 M = 33 10.1 / 31.4, 340 23.5 / 33.9, 1024 36.8 / 39.0, int8
+// with the dequant 6.7 / 25.0, 13.4 / 25.0, 22.3 / 25.3, to int32 at M = 512
+// 15.1 / 19.0 but 22.0 / 21.8 at 1024 (so that kind stops at 160 rows);
+// 12288x2048 SwiGLU bf16 M = 64 14.9 / 25.5, 128 19.6 / 29.1, 256 26.1 / 28.8;
+// 5120x2048 M = 256 13.8 / 15.9, 340 16.0 / 15.4; 8320x2048 M = 96 16.4 / 17.1,
+// 128 18.6 / 17.5 (wide outputs without SwiGLU stop at 160 rows too).
 void plan(int M, int N, int K, int kind, int* tile, int* splits) {
   const int es = kind_i8(kind) ? 1 : 2;
   const bool direct = kind == KIND_BF16 || kind == KIND_I32;
   *splits = 1;
+  const int rows = kind_swiglu(kind) ? 256 : kind == KIND_I32 || N > 4096 ? 160 : 192;
+  for (int c = 0; c < kKsTiles; ++c) {
+    if (kKsWeights[c] + kKsTokens[c] > rows) break;
+    if (kind_swiglu(kind) ? !kKsSwiglu[c] : !kKsPlain[c]) continue;
+    const int nc = kind_swiglu(kind) ? kKsWeights[c] / 2 : kKsWeights[c];
+    if ((long long)((M + kKsTokens[c] - 1) / kKsTokens[c]) * ((N + nc - 1) / nc) <= 256) {
+      *tile = kTiles + c;
+      return;
+    }
+  }
   if (kind_swiglu(kind)) {
     *tile = tiles_of(0, M, N, kind) >= 192 ? 0 : 3;
     return;
@@ -682,9 +677,19 @@ int launch_one(const GemmArgs& a, hipStream_t stream) {
   }
 }
 
+template <int FN, int FM, int W, int S, bool HALF, bool SWIGLU, bool PLAIN, int KIND>
+int launch_ks(const GemmArgs& a, hipStream_t stream) {
+  if constexpr (kind_swiglu(KIND) ? SWIGLU : PLAIN) return launch_ksplit<FN, FM, W, S, HALF, KIND>(a, stream);
+  else return (int)hipErrorInvalidValue;
+}
+
 template <int KIND>
 int launch_tile(int tile, const GemmArgs& a, hipStream_t stream) {
   switch (tile) {
+#define Q35_GEMM_KS_CASE(id, fn, fm, w, s, half, sg, pl) \
+  case kTiles + id: return launch_ks<fn, fm, w, s, half, sg, pl, KIND>(a, stream);
+    Q35_GEMM_KS_TILES(Q35_GEMM_KS_CASE)
+#undef Q35_GEMM_KS_CASE
 #define Q35_GEMM_CASE(id, wm, wn, fm, fn, rb, nsa, nsb, rot, staged) \
   case id: return launch_one<wm, wn, fm, fn, rb, nsa, nsb, rot, KIND, staged>(a, stream);
     Q35_GEMM_TILES(Q35_GEMM_CASE)
@@ -696,16 +701,18 @@ int launch_tile(int tile, const GemmArgs& a, hipStream_t stream) {
 int gemm_run(const void* A, const void* B, void* C, int M, int N, int K, int kind, const float* s_x,
              const float* s_w, int tile, int splits, void* ws, long long ws_bytes, hipStream_t stream) {
   Q35_CHECK_ARG(kind >= 0 && kind < kNumKinds);
-  if (tile < 0) plan(M, N, K, kind, &tile, &splits);
   const int es = kind_i8(kind) ? 1 : 2;
-  Q35_CHECK_ARG(A && B && C && M > 0 && N > 0 && K > 0);
-  Q35_CHECK_ARG(tile >= 0 && tile < kTiles && splits >= 1 && splits <= kMaxSplits);
-  Q35_CHECK_ARG(kStaged[tile] || kind == KIND_BF16 || kind == KIND_I32);
-  Q35_CHECK_ARG(q35_aligned16(A) && q35_aligned16(B) && ((long long)K * es) % kRB[tile] == 0);
+  Q35_CHECK_ARG(A && B && C && M > 0 && N > 0 && K > 0 && tile < kTiles);
+  if (tile < 0) plan(M, N, K, kind, &tile, &splits);
+  const bool ks = tile >= kTiles;
+  Q35_CHECK_ARG(splits >= 1 && splits <= kMaxSplits);
+  Q35_CHECK_ARG(ks || kStaged[tile] || kind == KIND_BF16 || kind == KIND_I32);
+  const int rb = ks ? 128 : kRB[tile];
+  Q35_CHECK_ARG(q35_aligned16(A) && q35_aligned16(B) && ((long long)K * es) % rb == 0);
   Q35_CHECK_ARG((kind != KIND_DEQ && kind != KIND_DEQ_SWIGLU) || (s_x && s_w));
   // 32-bit byte offsets of every operand row
   Q35_CHECK_ARG((long long)M * K * es < (1ll << 32) && (kind_swiglu(kind) ? 2ll : 1ll) * N * K * es < (1ll << 32));
-  const int nk = (int)((long long)K * es / kRB[tile]);
+  const int nk = (int)((long long)K * es / rb);
   Q35_CHECK_ARG(nk % splits == 0);
   if (splits > 1) {
     Q35_CHECK_ARG(kSplitOk[tile] && !kind_swiglu(kind) && tiles_of(tile, M, N, kind) <= kMaxSplitTiles);
@@ -733,8 +740,10 @@ extern "C" {
 // default plan); 0 when the plan does not split K, -1 for an invalid plan.
 long long q35_gemm_workspace(int M, int N, int K, int kind, int tile, int splits) {
   if (M <= 0 || N <= 0 || K <= 0 || kind < 0 || kind >= kNumKinds) return -1;
+  if (tile >= kTiles) return -1;
   if (tile < 0) plan(M, N, K, kind, &tile, &splits);
-  if (tile >= kTiles || splits < 1 || splits > kMaxSplits) return -1;
+  if (tile >= kTiles) return 0;
+  if (splits < 1 || splits > kMaxSplits) return -1;
   if (!kStaged[tile] && kind != KIND_BF16 && kind != KIND_I32) return -1;
   if (splits > 1 && (!kSplitOk[tile] || kind_swiglu(kind) || tiles_of(tile, M, N, kind) > kMaxSplitTiles))
     return -1;

@@ -1277,6 +1277,84 @@ def test_gemm_bf16_rejects_k():
         K.gemm_bf16(torch.zeros(4, 96, dtype=BF), torch.zeros(8, 96, dtype=BF))
 
 
+# (m, n, k) with the default plan on each tile of the K-splitting GEMM (few
+# tokens or columns), ragged in tokens and columns, one to many 128-byte pieces
+# of K per wave, and fewer pieces than waves
+_KS_SHAPES = [(2, 2048, 2048), (17, 2048, 6144), (65, 2045, 512), (100, 500, 1152), (33, 5120, 2048),
+              (97, 5116, 256), (129, 2048, 640), (150, 5120, 128), (200, 2000, 6144), (340, 2048, 384),
+              (500, 2044, 1024), (256, 5100, 2048), (784, 2048, 256), (1000, 1152, 512), (95, 8320, 2048)]
+
+
+@pytest.mark.parametrize("m,n,k", _KS_SHAPES)
+def test_gemm_ksplit_bf16(gpu, m, n, k):
+    """bf16 GEMM of few tokens or columns, waves splitting K: against the fp64
+    product (one bf16 rounding plus the fp32 sum of k terms), the same bits on
+    a repeated launch, no write past the output."""
+    from ppu_amd import kernels as K
+
+    g = gen(KERNEL_SEED + 97)
+    w, x = randn(g, n, k, scale=0.02), randn(g, m, k)
+    xd, wd = x.to(gpu), w.to(gpu)
+    y = torch.full((m + 1, n), 7.0, dtype=BF, device=gpu)
+    K.gemm_into(xd, wd, y[:m], K.GEMM_BF16)
+    ref = xd.double() @ wd.double().t()
+    # |error| <= half a bf16 ulp of the result + k * 2^-24 of the sum of |terms|
+    bound = ref.abs() * 2.0**-8 + k * 2.0**-24 * (xd.double().abs() @ wd.double().abs().t()) + 1e-30
+    assert bool(((y[:m].double() - ref).abs() <= bound).all())
+    assert bool((y[m] == 7.0).all())
+    y2 = torch.empty(m, n, dtype=BF, device=gpu)
+    assert torch.equal(K.gemm_into(xd, wd, y2, K.GEMM_BF16), y[:m])
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 6144, 2048), (64, 6144, 128), (90, 6100, 2048), (128, 6144, 256),
+                                   (150, 6144, 2048), (256, 6140, 512), (5, 24, 192)])
+def test_gemm_ksplit_swiglu(gpu, m, n, k):
+    """The SwiGLU kinds on the K-splitting tiles: bf16 against the fp64 product
+    of bf16-rounded gate and up, int8 bit-equal to the int32 accumulators
+    dequantised, rounded and combined by the separate kernels."""
+    from ppu_amd import kernels as K
+
+    g = gen(KERNEL_SEED + 98)
+    w, x = randn(g, 2 * n, k, scale=0.02).to(gpu), randn(g, m, k).to(gpu)
+    y = K.gemm_bf16(x, w, swiglu=True)
+    acc = x.double() @ w.double().t()
+    gate, up = acc[:, :n], acc[:, n:]
+    exp = torch.nn.functional.silu(gate) * up
+    # four bf16 roundings (gate, up, silu, product); |silu'| <= 1.1
+    bound = 2.0**-8 * (1.1 * gate.abs() * up.abs() + 3 * exp.abs()) * 1.05 + 1e-6
+    assert bool(((y.double() - exp).abs() <= bound).all())
+    wq, sw = K.quantize_weight_i8(w)
+    xq, sx = K.quantize_act_i8(x)
+    if k % 128 == 0:
+        got = K.gemm_a8w8(xq, sx, wq, sw, swiglu=True)
+        acc = (xq.cpu().double() @ wq.cpu().double().t())
+        deq = oa.dequant(acc.numpy().astype(np.int32), sx.cpu().numpy(), sw.cpu().numpy())
+        assert torch.equal(got, K.silu_and_mul(deq.to(gpu).contiguous()))
+
+
+@pytest.mark.parametrize("m,n,k", [s for s in _KS_SHAPES if s[2] % 128 == 0])
+def test_gemm_ksplit_int8_exact(gpu, m, n, k):
+    """int8 kinds on the K-splitting tiles: int32 accumulators and the dequant
+    bit-exact, in three graph replays too."""
+    from ppu_amd import kernels as K
+
+    g = gen(KERNEL_SEED + 99)
+    wq, sw = K.quantize_weight_i8(randn(g, n, k, scale=0.02).to(gpu))
+    xq, sx = K.quantize_act_i8(randn(g, m, k).to(gpu))
+    exact = _exact_i8_product(xq, wq)
+    assert torch.equal(K.a8w8_int_gemm(xq, wq).cpu().to(torch.int64), exact)
+    y = K.gemm_a8w8(xq, sx, wq, sw)
+    assert torch.equal(y.cpu(), oa.dequant(exact.numpy().astype(np.int32), sx.cpu().numpy(), sw.cpu().numpy()))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y2 = K.gemm_a8w8(xq, sx, wq, sw)
+    for _ in range(3):
+        y2.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y2, y)
+
+
 @pytest.mark.parametrize("m", [3, 8, 16])
 @pytest.mark.parametrize("n,k", [(12288, 2048), (2048, 6144)])
 def test_a8w8_prequantised_abi(gpu, m, n, k):
