@@ -898,6 +898,30 @@ def test_prefill_attention_groupings(gpu, q_heads, kv_heads):
     assert torch.equal(got_s, got)
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,seq_len,start,cache", [
+    (8, 2, 1, 0, 64), (8, 2, 31, 33, 64), (8, 2, 32, 0, 32), (8, 2, 33, 64, 512), (8, 2, 65, 63, 200),
+    (8, 2, 17, 3000, 3200), (2, 2, 129, 0, 129), (2, 2, 40, 700, 1024), (4, 2, 97, 5, 160),
+    (8, 1, 70, 300, 512), (16, 2, 45, 0, 64), (8, 2, 2100, 0, 2176)])
+@pytest.mark.parametrize("spread", [1.0, 6.0])
+def test_prefill_attention_tiles(gpu, q_heads, kv_heads, seq_len, start, cache, spread):
+    """Edges of the 32-row tiles and 64-key blocks, ranges of one to many
+    blocks, every head grouping, batch 2, NaN behind the valid end; ``spread``
+    widens the scores so that row maxima keep moving (rescales)."""
+    from ppu_amd import kernels as K
+
+    g = gen(KERNEL_SEED + 25)
+    batch = 2 if seq_len < 100 else 1
+    q = randn(g, batch, q_heads, seq_len, 256, scale=spread)
+    kc = randn(g, batch, kv_heads, cache, 256)
+    vc = randn(g, batch, kv_heads, cache, 256)
+    exp = ref.prefill_attention(q, kc, vc, 0.0625, start)
+    kg, vg = kc.to(gpu), vc.to(gpu)
+    kg[:, :, start + seq_len:] = float("nan")
+    vg[:, :, start + seq_len:] = float("inf")
+    got = K.gqa_prefill_attention(q.to(gpu), kg, vg, 0.0625, kv_start=start)
+    close(got, exp)
+
+
 @pytest.mark.parametrize("q_heads,kv_heads", [(8, 2), (4, 2)])
 def test_prefill_attention_split_keys(gpu, q_heads, kv_heads):
     """Query tiles with more than 4 key blocks of 64 split their key range over
