@@ -435,7 +435,7 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
     constexpr int ITER = PR * CPRW / 256;      // chunks per thread and phase
     constexpr int SCO = PR * SB;               // LDS offset of the scales
     static_assert(PR * CPRW % 256 == 0, "the chunks divide over the workgroup");
-    static_assert(SCO + NSC * 4 <= LDSB, "the staged tile and scales fit the rings");
+    static_assert(!STAGED || SCO + NSC * 4 <= LDSB, "the staged tile and scales fit the rings");
     const bool vec = (a.N & 7) == 0;
     float* sc = reinterpret_cast<float*>(lds + SCO);
     wait_lds();
@@ -541,6 +541,12 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
 //   5: tile 0 with direct stores; 6: tile 1 with direct stores; 7: tile 6
 //   without K rotation
 //   8: 128 x 64 (2 x 1), RB 128, NSA 6, NSB 8, rot, direct   (160 KiB)
+//   9: 256 x 256 (4 x 4), RB 128, NSA 2, NSB 3, staged; 10: direct (160 KiB;
+//   picked by the default plan only). 16 MFMAs for 8 fragment reads per k step
+//   (12 for 7 in tile 0): the most work per LDS byte, for outputs that fill
+//   their last round of CUs with it: 2048x6144 bf16 at 8192 tokens 222 -> 175
+//   us (1180 TFLOP/s), 12288x2048 SwiGLU at 4096 204 -> 191 us, int8 2048x6144
+//   at 8192 128 -> 99 us (2080 TOP/s)
 #define Q35_GEMM_TILES(X)                     \
   X(0, 2, 2, 4, 3, 128, 2, 4, false, true)    \
   X(1, 2, 2, 2, 2, 128, 4, 6, true, true)     \
@@ -550,13 +556,16 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
   X(5, 2, 2, 4, 3, 128, 2, 4, false, false)   \
   X(6, 2, 2, 2, 2, 128, 4, 6, true, false)    \
   X(7, 2, 2, 2, 2, 128, 4, 6, false, false)   \
-  X(8, 2, 2, 2, 1, 128, 6, 8, true, false)
-constexpr int kTiles = 9;
-constexpr int kTM[kTiles] = {256, 128, 256, 128, 256, 256, 128, 128, 128};
-constexpr int kTN[kTiles] = {192, 128, 128, 192, 192, 192, 128, 128, 64};
-constexpr int kRB[kTiles] = {128, 128, 128, 128, 128, 128, 128, 128, 128};
-constexpr bool kStaged[kTiles] = {true, true, true, true, true, false, false, false, false};
-constexpr bool kSplitOk[kTiles] = {false, true, true, true, false, false, true, true, true};  // up to 8 blocks per wave
+  X(8, 2, 2, 2, 1, 128, 6, 8, true, false)    \
+  X(9, 2, 2, 4, 4, 128, 2, 3, false, true)    \
+  X(10, 2, 2, 4, 4, 128, 2, 3, false, false)
+constexpr int kTiles = 11;
+constexpr int kPlanTiles = 9;  // tiles a caller's plan may name
+constexpr int kRB = 128;
+constexpr int kTM[kTiles] = {256, 128, 256, 128, 256, 256, 128, 128, 128, 256, 256};
+constexpr int kTN[kTiles] = {192, 128, 128, 192, 192, 192, 128, 128, 64, 256, 256};
+constexpr bool kStaged[kTiles] = {true, true, true, true, true, false, false, false, false, true, false};
+constexpr bool kSplitOk[kTiles] = {false, true, true, true, false, false, true, true, true, false, false};  // up to 8 blocks per wave
 constexpr int kMaxSplits = 8;
 
 // Tiles of the K-splitting kernel, by operand rows (32 FN weight rows, 16 for
@@ -600,29 +609,51 @@ long long workspace_bytes(int tile, int M, int N, int kind, int splits) {
   return kCounterBytes + tiles_of(tile, M, N, kind) * splits * kTM[tile] * kTN[tile] * 4ll;
 }
 
-// Default plan by output shape (measured at M = 1024 on the 2B prefill
-// shapes, profiles/prefill_gemm_sweep.txt): the widest tile that still gives
-// most CUs a workgroup, with direct stores for the bf16 / int32 kinds and the
-// staged epilogue for SwiGLU and dequant; outputs with fewer tiles than CUs
-// split K only when each split keeps at least 40 stages (the partial-tile
-// exchange costs more than the idle CUs below that).
+// Time of one workgroup of a ring tile with all CUs busy: kFixed + kStage per
+// stage of 128 bytes, in us (fits of outputs 2048 to 12288 wide with K = 2048
+// and 6144 bf16 or int8; by tile, 1 and 6, 0 and 5, 9 and 10 alike). kDequant:
+// what the dequant epilogue adds (9 also with SwiGLU, about half).
+constexpr double kFixed[kTiles] = {11.6, 5.7, 7, 7.7, 11.6, 11.6, 5.7, 5.7, 4.8, 5.1, 5.1};
+constexpr double kStage[kTiles] = {1.06, 0.51, 0.92, 0.667, 1.06, 1.06, 0.51, 0.51, 0.353, 1.7, 1.7};
+constexpr double kDequant[kTiles] = {0, 1.3, 2, 0.5, 0, 0, 0, 0, 0, 10, 0};
+
+// Estimated time of an output on a ring tile: whole rounds of 256 workgroups,
+// and a last one that costs 0.7 of a round even if few CUs take part (0.45
+// where earlier rounds have spread the workgroups' ends).
+double ring_us(int tile, int M, int N, int nk, int kind) {
+  const double r = (double)tiles_of(tile, M, N, kind) / 256;
+  const double one = kFixed[tile] + kStage[tile] * nk +
+                     kDequant[tile] * (kind == KIND_DEQ ? 1 : kind == KIND_DEQ_SWIGLU && tile == 9 ? 0.45 : 0);
+  if (r <= 1) return one * (0.7 + 0.3 * r);
+  const double whole = (double)(long long)r, rest = r - whole;
+  return one * (whole + (rest > 0 ? (whole < 3 ? 0.7 + 0.3 * rest : 0.45 + 0.5 * rest) : 0));
+}
+
+// Default plan. Large outputs: the ring tile with the least estimated time,
+// direct stores for the bf16 / int32 kinds and the staged epilogue for SwiGLU
+// and dequant. What it decides is the last round of CUs: the down projection
+// (2048x6144) at 4096 tokens has 176 tiles of 256x192 (116 us) but 256 of
+// 256x128 (95 us), at 2003 tokens 66 us on 256x192 and 54 us on 128x128. Outputs
+// with fewer 128x128 tiles than CUs split K only when each split keeps at least
+// 40 stages (the partial-tile exchange costs more than the idle CUs below that).
 //
 // Outputs of few tokens or few columns run on the K-splitting kernel instead
 // (tile kTiles + its index): the smallest of its tiles that covers the output
 // with one workgroup per CU, as long as the tile's operand rows stay few
 // enough. Measured at the edges (us, this kernel against the ring plans, cold
-// weights): 2048x2048 bf16 M = 33 5.4 / 13.5, 340 9.9 / 13.8, 1024 15.0 / 14.9;
-// 2048x6144 bf16 M = 33 10.1 / 31.4, 340 23.5 / 33.9, 1024 36.8 / 39.0, int8
-// with the dequant 6.7 / 25.0, 13.4 / 25.0, 22.3 / 25.3, to int32 at M = 512
-// 15.1 / 19.0 but 22.0 / 21.8 at 1024 (so that kind stops at 160 rows);
-// 12288x2048 SwiGLU bf16 M = 64 14.9 / 25.5, 128 19.6 / 29.1, 256 26.1 / 28.8;
-// 5120x2048 M = 256 13.8 / 15.9, 340 16.0 / 15.4; 8320x2048 M = 96 16.4 / 17.1,
-// 128 18.6 / 17.5 (wide outputs without SwiGLU stop at 160 rows too).
+// weights): 2048x2048 bf16 M = 33 5.4 / 13.5, 340 9.9 / 13.8, 600 12.1 / 13.0,
+// 1024 (192 rows) 14.8 / 13.8; 2048x6144 bf16 M = 33 10.1 / 31.4, 340 23.5 /
+// 33.9, 600 30.2 / 35.0; int8 with the dequant M = 33 6.7 / 25.0, 340 13.4 /
+// 25.0, 1024 (192 rows) 22.2 / 24.9, to int32 at 512 15.1 / 19.0, at 1024 20.2 /
+// 20.1; 5120x2048 M = 256 13.8 / 15.9, 340 (192 rows) 16.0 / 15.4; 8320x2048 M =
+// 96 16.4 / 17.1, 128 (192 rows) 18.6 / 17.5; 12288x2048 SwiGLU bf16 M = 64 14.9 /
+// 25.5, 128 19.6 / 29.1, 230 (256 rows) 25.5 / 26.9, int8 180 (224 rows) 15.9 /
+// 16.7, 230 (256 rows) 18.4 / 16.9.
 void plan(int M, int N, int K, int kind, int* tile, int* splits) {
   const int es = kind_i8(kind) ? 1 : 2;
   const bool direct = kind == KIND_BF16 || kind == KIND_I32;
   *splits = 1;
-  const int rows = kind_swiglu(kind) ? 256 : kind == KIND_I32 || N > 4096 ? 160 : 192;
+  const int rows = kind == KIND_SWIGLU ? 256 : kind == KIND_DEQ_SWIGLU ? 224 : kind == KIND_DEQ && N <= 4096 ? 192 : 160;
   for (int c = 0; c < kKsTiles; ++c) {
     if (kKsWeights[c] + kKsTokens[c] > rows) break;
     if (kind_swiglu(kind) ? !kKsSwiglu[c] : !kKsPlain[c]) continue;
@@ -632,23 +663,21 @@ void plan(int M, int N, int K, int kind, int* tile, int* splits) {
       return;
     }
   }
-  if (kind_swiglu(kind)) {
-    *tile = tiles_of(0, M, N, kind) >= 192 ? 0 : 3;
-    return;
+  const int nk = (int)((long long)K * es / kRB);
+  double best = 0;
+  *tile = -1;
+  for (int t = 0; t < kTiles; ++t) {
+    // 4 and 7 are tiles 0 and 6 with another ring or walk: never faster
+    if (t == 4 || t == 7 || (direct ? t == 0 || t == 1 || t == 9 : !kStaged[t])) continue;
+    if (kind_swiglu(kind) && (t == 1 || t == 2)) continue;  // few columns per tile: the epilogue outweighs
+    const double us = ring_us(t, M, N, nk, kind);
+    if (*tile < 0 || us < best) {
+      best = us;
+      *tile = t;
+    }
   }
-  if (tiles_of(0, M, N, kind) >= 160) {
-    *tile = direct ? 5 : 0;
-  } else if (tiles_of(3, M, N, kind) >= 160) {
-    *tile = 3;
-  } else if (direct && tiles_of(8, M, N, kind) <= 256) {
-    // one round of 128x64 tiles: at M = 1024, N = 2048 all 256 CUs without a
-    // K split (o_proj 18.4 -> 14.8 us, down 44.9 -> 37.9 us against 128x128
-    // tiles on 128 CUs, split 2 for the down projection)
-    *tile = 8;
-  } else {
-    *tile = direct ? 6 : 1;
+  if (*tile == 1 || *tile == 6) {
     const long long t = tiles_of(1, M, N, kind);
-    const int nk = K * es / kRB[1];
     while (*splits < kMaxSplits && t * *splits * 2 <= 256 && nk % (*splits * 2) == 0 &&
            nk / (*splits * 2) >= 40 && t <= kMaxSplitTiles)
       *splits *= 2;
@@ -702,17 +731,16 @@ int gemm_run(const void* A, const void* B, void* C, int M, int N, int K, int kin
              const float* s_w, int tile, int splits, void* ws, long long ws_bytes, hipStream_t stream) {
   Q35_CHECK_ARG(kind >= 0 && kind < kNumKinds);
   const int es = kind_i8(kind) ? 1 : 2;
-  Q35_CHECK_ARG(A && B && C && M > 0 && N > 0 && K > 0 && tile < kTiles);
+  Q35_CHECK_ARG(A && B && C && M > 0 && N > 0 && K > 0 && tile < kPlanTiles);
   if (tile < 0) plan(M, N, K, kind, &tile, &splits);
   const bool ks = tile >= kTiles;
   Q35_CHECK_ARG(splits >= 1 && splits <= kMaxSplits);
   Q35_CHECK_ARG(ks || kStaged[tile] || kind == KIND_BF16 || kind == KIND_I32);
-  const int rb = ks ? 128 : kRB[tile];
-  Q35_CHECK_ARG(q35_aligned16(A) && q35_aligned16(B) && ((long long)K * es) % rb == 0);
+  Q35_CHECK_ARG(q35_aligned16(A) && q35_aligned16(B) && ((long long)K * es) % kRB == 0);
   Q35_CHECK_ARG((kind != KIND_DEQ && kind != KIND_DEQ_SWIGLU) || (s_x && s_w));
   // 32-bit byte offsets of every operand row
   Q35_CHECK_ARG((long long)M * K * es < (1ll << 32) && (kind_swiglu(kind) ? 2ll : 1ll) * N * K * es < (1ll << 32));
-  const int nk = (int)((long long)K * es / rb);
+  const int nk = (int)((long long)K * es / kRB);
   Q35_CHECK_ARG(nk % splits == 0);
   if (splits > 1) {
     Q35_CHECK_ARG(kSplitOk[tile] && !kind_swiglu(kind) && tiles_of(tile, M, N, kind) <= kMaxSplitTiles);
@@ -740,7 +768,7 @@ extern "C" {
 // default plan); 0 when the plan does not split K, -1 for an invalid plan.
 long long q35_gemm_workspace(int M, int N, int K, int kind, int tile, int splits) {
   if (M <= 0 || N <= 0 || K <= 0 || kind < 0 || kind >= kNumKinds) return -1;
-  if (tile >= kTiles) return -1;
+  if (tile >= kPlanTiles) return -1;
   if (tile < 0) plan(M, N, K, kind, &tile, &splits);
   if (tile >= kTiles) return 0;
   if (splits < 1 || splits > kMaxSplits) return -1;

@@ -1301,6 +1301,32 @@ def test_gemm_bf16_rejects_k():
         K.gemm_bf16(torch.zeros(4, 96, dtype=BF), torch.zeros(8, 96, dtype=BF))
 
 
+# (m, n, k) whose default plan is the 256x256 ring tile (whole rounds of it),
+# ragged in tokens and columns
+@pytest.mark.parametrize("m,n,k", [(4000, 4090, 256), (8100, 2048, 192)])
+def test_gemm_256_tile(gpu, m, n, k):
+    """The widest ring tile, chosen by the default plan only: bf16 (direct) and
+    SwiGLU (staged) against fp64, int8 kinds bit-exact."""
+    from ppu_amd import kernels as K
+
+    g = gen(KERNEL_SEED + 96)
+    w, x = randn(g, n, k, scale=0.05).to(gpu), randn(g, m, k).to(gpu)
+    ref = x.double() @ w.double().t()
+    bound = ref.abs() * 2.0**-8 + k * 2.0**-24 * (x.double().abs() @ w.double().abs().t()) + 1e-30
+    assert bool(((K.gemm_bf16(x, w).double() - ref).abs() <= bound).all())
+    gate, up = ref[:, : n // 2], ref[:, n // 2 :]
+    exp = torch.nn.functional.silu(gate) * up
+    bound = 2.0**-8 * (1.1 * gate.abs() * up.abs() + 3 * exp.abs()) * 1.05 + 1e-6
+    assert bool(((K.gemm_bf16(x, w, swiglu=True).double() - exp).abs() <= bound).all())
+    if k % 128 == 0:
+        wq, sw = K.quantize_weight_i8(w)
+        xq, sx = K.quantize_act_i8(x)
+        acc = (xq.double() @ wq.double().t()).to(torch.int64)  # exact: |sum| < 2^53
+        assert torch.equal(K.a8w8_int_gemm(xq, wq).to(torch.int64), acc)
+        deq = (acc.float() * sx.view(-1, 1) * sw.view(1, -1)).to(BF)
+        assert torch.equal(K.gemm_a8w8(xq, sx, wq, sw), deq)
+
+
 # (m, n, k) with the default plan on each tile of the K-splitting GEMM (few
 # tokens or columns), ragged in tokens and columns, one to many 128-byte pieces
 # of K per wave, and fewer pieces than waves
