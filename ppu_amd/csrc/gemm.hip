@@ -72,8 +72,11 @@
 //
 // Tile order: units (tile, split) are grouped so that the units sharing B
 // rows and a K range (consecutive M tiles) run on one XCD and read the
-// weights into one L2: with U units and U % 8 == 0, workgroup b (XCD b % 8)
-// takes unit (b % 8) * U / 8 + b / 8, M tile fastest.
+// weights into one L2: workgroup b (XCD b % 8) takes the b / 8-th of the XCD's
+// eighth of the units. M runs fastest within bands of 8 M tiles, so the 32
+// units that an XCD works on at a time are 8 M tiles x 4 N tiles and share both
+// operands (with all M tiles fastest, each XCD of 2048x6144 at 8192 tokens
+// streamed all 100 MB of activations for one N tile).
 #include "gemm_ksplit.hpp"
 
 namespace {
@@ -92,6 +95,8 @@ Q35_DEV uint32_t acc_bits(float v) { return __float_as_uint(v); }
 Q35_DEV uint32_t acc_bits(int v) { return (uint32_t)v; }
 Q35_DEV float acc_from(uint32_t b, float) { return __uint_as_float(b); }
 Q35_DEV int acc_from(uint32_t b, int) { return (int)b; }
+
+constexpr int kBand = 8;
 
 template <bool V> struct BoolTag { static constexpr bool value = V; };
 
@@ -114,6 +119,12 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
   constexpr int NMF = FM * FN;               // MFMAs per k step
   constexpr int NR = FM + FN;                // fragment reads per k step
   constexpr int H = NMF / 2;                 // MFMAs of the last step before the barrier
+  // MFMA slots that carry the DMA refills, spread evenly: four waves issuing
+  // one 1 KiB copy per 32-cycle MFMA ask the texture unit for twice its 64
+  // bytes per clock, and the MFMAs stall behind the copies (one copy per slot
+  // from the first on: 8320x2048 bf16 at 1024 tokens 39.0 us, spread 35.8;
+  // SwiGLU 12288x2048 at 4096 175 -> 168 us)
+  constexpr int SLOTS = (T - 1) * NMF;
   static_assert(WM * WN == 4, "4 waves");
   static_assert(GA % 4 == 0 && GB % 4 == 0, "every wave issues the same DMA groups of A and B");
   static_assert(T % 2 == 0, "fragment register sets alternate between k steps");
@@ -136,10 +147,14 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
   const int ntiles = mt * nt;
   const int S = SPLIT ? a.splits : 1;
   const int U = ntiles * S;
-  int u = (int)blockIdx.x;
-  if ((U & 7) == 0) u = (u & 7) * (U >> 3) + (u >> 3);
-  const int tm = u % mt;
-  const int rest = u / mt;
+  const int xcd = (int)blockIdx.x & 7;
+  int u = xcd * (U >> 3) + min(xcd, U & 7) + ((int)blockIdx.x >> 3);
+  // bands of kBand M tiles (the last one smaller): M tile fastest inside one
+  const int band = u / (kBand * nt * S);
+  u -= band * (kBand * nt * S);
+  const int bm = min(kBand, mt - band * kBand);
+  const int tm = band * kBand + u % bm;
+  const int rest = u / bm;
   const int ks = SPLIT ? rest % S : 0;
   const int tn = SPLIT ? rest / S : rest;
   const int tile = tn * mt + tm;
@@ -276,8 +291,11 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
           for (int r = q * NR / NMF; r < (q + 1) * NR / NMF; ++r) read1(abuf, bbuf, t + 1, (t + 1) & 1, r);
         }
         const int slot = t * NMF + q;
-        if (RA && slot < LA) dma(kt + NSA - 1, rabuf, 0, slot);
-        if (RB_ && slot >= LA && slot < LPW) dma(kt + NSB - 1, 0, rbbuf, slot);
+        const int i = (slot * LPW + SLOTS - 1) / SLOTS;  // the copy at slot i * SLOTS / LPW
+        if (i < LPW && i * SLOTS / LPW == slot) {
+          if (RA && i < LA) dma(kt + NSA - 1, rabuf, 0, i);
+          if (RB_ && i >= LA) dma(kt + NSB - 1, 0, rbbuf, i);
+        }
         Q35_PIN();
       }
     }
