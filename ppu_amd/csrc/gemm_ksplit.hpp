@@ -90,9 +90,10 @@ __global__ __launch_bounds__(W * 64) void gemm_ksplit(const GemmArgs a) {
   const int mt = (a.M + TM - 1) / TM;
   const int nt = (a.N + NC - 1) / NC;
   const int U = mt * nt;
-  int u = (int)blockIdx.x;
-  // consecutive units (the M tiles of one weight tile) on one XCD
-  if ((U & 7) == 0) u = (u & 7) * (U >> 3) + (u >> 3);
+  // consecutive units (the M tiles of one weight tile) on one XCD: workgroup b
+  // (XCD b % 8) takes the b / 8-th of the XCD's eighth of the units
+  const int xcd = (int)blockIdx.x & 7;
+  const int u = xcd * (U >> 3) + min(xcd, U & 7) + ((int)blockIdx.x >> 3);
   const int m0 = (u % mt) * TM, n0 = (u / mt) * NC;
   const uint32_t rowb = (uint32_t)a.K * ES;
   const int np = (int)(rowb >> 7);                   // pieces of a row
