@@ -412,6 +412,14 @@ int q35_gemm(const void* A, const void* B, void* C, int M, int N, int K, int kin
              const void* s_w, int tile, int splits, void* workspace, long long workspace_bytes,
              void* stream);
 
+/* C[M, N] = bf16(A . B^T + bias) (A [M, K], B [N, K], bias [N], all bf16), or
+ * with gelu the tanh-approximated GELU of the sum, both on the fp32
+ * accumulators: F.linear with a bias, and fc1 -> GELU, of the vision tower
+ * (integration.py:514-562, 644-735). K % 64 == 0; A and B 16-byte aligned. No
+ * counterpart among the reference's kernels. */
+int q35_gemm_bias(const void* A, const void* B, const void* bias, void* C, int M, int N, int K,
+                  int gelu, void* stream);
+
 /* A8W8 prefill between the int8 GEMMs of a layer: residual add of the
  * dequantised accumulators of the previous GEMM (q35_dequant_i32's values) +
  * RMSNorm (width 2048, (1 + w) weight) with the normalised rows quantised per

@@ -7,6 +7,7 @@
 //   kind 2  int8 A, B -> int32 C = acc (exact)                     [the int8 GEMM of explore_runtime_quantization.py:173-180]
 //   kind 3  int8 -> bf16 C = bf16(float(acc) * s_x[m] * s_w[n])    [the same with its dequant]
 //   kind 4  int8, B = [gate; up] -> SwiGLU of the dequantised gate and up (kind 1's rounding points)
+//   q35_gemm_bias  bf16 -> bf16(acc + bias[n]), or of its tanh GELU   [the vision tower's F.linear]
 //
 // bf16 runs on v_mfma_f32_32x32x16_bf16 (fp32 accumulators), int8 on
 // v_mfma_i32_32x32x32_i8 (exact int32). Both take 16 bytes per lane and
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
   static_assert(!SWIGLU || WN == 2, "SwiGLU pairs the gate waves with the up waves");
   static_assert(NSA >= 2 && NSB >= NSA && LDSB <= 160 * 1024, "the stage rings fit the LDS");
   static_assert(LPW <= (T - 1) * NMF, "the refill fits the MFMA slots of the first steps");
-  static_assert(STAGED || KIND == KIND_BF16 || KIND == KIND_I32, "direct stores: bf16 and int32 kinds");
+  static_assert(STAGED || kind_direct(KIND), "direct stores: bf16 and int32 kinds");
   using AccT = typename GemmAcc<I8>::T;
   using EltT = typename GemmAcc<I8>::E;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[LDSB];
@@ -403,13 +404,24 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
     const int rbase = m0 + wm * FM * 32 + 4 * kh;
     const int cbase = n0 + wn * FN * 32 + l32;
     const bool full = m0 + TM <= a.M && n0 + TN <= a.N;
+    float bias[FN];
+    if constexpr (kind_bias(KIND)) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) bias[j] = bias_at(a, min(cbase + 32 * j, a.N - 1));
+    }
     auto store = [&](int i, int r, int j, bool check) {
       const int row = rbase + 32 * i + 8 * (r >> 2) + (r & 3);
       const int col = cbase + 32 * j;
       if (check && (row >= a.M || col >= a.N)) return;
       const size_t at = (size_t)row * a.N + col;
-      if constexpr (KIND == KIND_I32) reinterpret_cast<int*>(a.C)[at] = acc[i][j][r];
-      else reinterpret_cast<uint16_t*>(a.C)[at] = (uint16_t)f2bf(acc[i][j][r]);
+      if constexpr (KIND == KIND_I32) {
+        reinterpret_cast<int*>(a.C)[at] = acc[i][j][r];
+      } else {
+        float v = acc[i][j][r];
+        if constexpr (kind_bias(KIND)) v += bias[j];
+        if constexpr (KIND == KIND_BIAS_GELU) v = gelu_tanh_fast(v);
+        reinterpret_cast<uint16_t*>(a.C)[at] = (uint16_t)f2bf(v);
+      }
     };
     if (full) {
 #pragma unroll
@@ -475,6 +487,9 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
         if constexpr (DEQ) {
 #pragma unroll
           for (int j = 0; j < FN; ++j) swr[j] = sc[TM + wn * FN * 32 + j * 32 + l32];
+        } else if constexpr (kind_bias(KIND)) {
+#pragma unroll
+          for (int j = 0; j < FN; ++j) swr[j] = bias_at(a, min(n0 + wn * FN * 32 + j * 32 + l32, a.N - 1));
         }
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
@@ -493,6 +508,10 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
               if constexpr (DEQ) {
                 const float d = (float)acc[i][j][r] * sxr[r >> 2][r & 3] * swr[j];
                 *reinterpret_cast<uint16_t*>(lds + off) = (uint16_t)f2bf(d);
+              } else if constexpr (kind_bias(KIND)) {
+                const float v = acc[i][j][r] + swr[j];
+                *reinterpret_cast<uint16_t*>(lds + off) =
+                    (uint16_t)f2bf(KIND == KIND_BIAS_GELU ? gelu_tanh_fast(v) : v);
               } else if constexpr (W16)
                 *reinterpret_cast<uint16_t*>(lds + off) = (uint16_t)f2bf(acc[i][j][r]);
               else
@@ -522,7 +541,7 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
           int* C = reinterpret_cast<int*>(a.C) + at;
           if (vec && ncol == VPC) *reinterpret_cast<q35_u32x4*>(C) = v[it];
           else for (int e = 0; e < ncol; ++e) C[e] = (int)v[it][e];
-        } else if constexpr (KIND == KIND_BF16 || KIND == KIND_DEQ) {
+        } else if constexpr (!SWIGLU) {
           uint16_t* C = reinterpret_cast<uint16_t*>(a.C) + at;
           if (vec && ncol == VPC) *reinterpret_cast<q35_u32x4*>(C) = v[it];
           else for (int e = 0; e < ncol; ++e) C[e] = (uint16_t)(v[it][e >> 1] >> (16 * (e & 1)));
@@ -669,7 +688,7 @@ double ring_us(int tile, int M, int N, int nk, int kind) {
 // 16.7, 230 (256 rows) 18.4 / 16.9.
 void plan(int M, int N, int K, int kind, int* tile, int* splits) {
   const int es = kind_i8(kind) ? 1 : 2;
-  const bool direct = kind == KIND_BF16 || kind == KIND_I32;
+  const bool direct = kind_direct(kind);
   *splits = 1;
   const int rows = kind == KIND_SWIGLU ? 256 : kind == KIND_DEQ_SWIGLU ? 224 : kind == KIND_DEQ && N <= 4096 ? 192 : 160;
   for (int c = 0; c < kKsTiles; ++c) {
@@ -694,7 +713,7 @@ void plan(int M, int N, int K, int kind, int* tile, int* splits) {
       *tile = t;
     }
   }
-  if (*tile == 1 || *tile == 6) {
+  if ((*tile == 1 || *tile == 6) && !kind_bias(kind)) {
     const long long t = tiles_of(1, M, N, kind);
     while (*splits < kMaxSplits && t * *splits * 2 <= 256 && nk % (*splits * 2) == 0 &&
            nk / (*splits * 2) >= 40 && t <= kMaxSplitTiles)
@@ -704,7 +723,7 @@ void plan(int M, int N, int K, int kind, int* tile, int* splits) {
 
 template <int WM, int WN, int FM, int FN, int RB, int NSA, int NSB, bool ROT, int KIND, bool STAGED>
 int launch_one(const GemmArgs& a, hipStream_t stream) {
-  if constexpr (!STAGED && KIND != KIND_BF16 && KIND != KIND_I32) {
+  if constexpr (!STAGED && !kind_direct(KIND)) {
     return (int)hipErrorInvalidValue;  // direct stores: bf16 and int32 kinds
   } else {
   constexpr int TM = WM * FM * 32, TN = WN * FN * 32;
@@ -712,7 +731,7 @@ int launch_one(const GemmArgs& a, hipStream_t stream) {
   const long long units = (long long)((a.M + TM - 1) / TM) * ((a.N + NC - 1) / NC) * a.splits;
   Q35_CHECK_ARG(units < (1ll << 31));
   if (a.splits > 1) {
-    if constexpr (kind_swiglu(KIND) || FM * FN > 8) {
+    if constexpr (kind_swiglu(KIND) || kind_bias(KIND) || FM * FN > 8) {
       return (int)hipErrorInvalidValue;  // split K: tiles of up to 8 blocks per wave, no SwiGLU
     } else {
       gemm_ring<WM, WN, FM, FN, RB, NSA, NSB, ROT, KIND, true, STAGED><<<(unsigned)units, 256, 0, stream>>>(a);
@@ -732,6 +751,14 @@ int launch_ks(const GemmArgs& a, hipStream_t stream) {
 
 template <int KIND>
 int launch_tile(int tile, const GemmArgs& a, hipStream_t stream) {
+  if constexpr (kind_bias(KIND)) {
+    // q35_gemm_bias has the default plan only: the tiles it takes for the direct
+    // kinds, unsplit
+    switch (tile) {
+      case 0: case 1: case 4: case 7: case 9: return (int)hipErrorInvalidValue;
+      default: break;
+    }
+  }
   switch (tile) {
 #define Q35_GEMM_KS_CASE(id, fn, fm, w, s, half, sg, pl) \
   case kTiles + id: return launch_ks<fn, fm, w, s, half, sg, pl, KIND>(a, stream);
@@ -747,13 +774,12 @@ int launch_tile(int tile, const GemmArgs& a, hipStream_t stream) {
 
 int gemm_run(const void* A, const void* B, void* C, int M, int N, int K, int kind, const float* s_x,
              const float* s_w, int tile, int splits, void* ws, long long ws_bytes, hipStream_t stream) {
-  Q35_CHECK_ARG(kind >= 0 && kind < kNumKinds);
   const int es = kind_i8(kind) ? 1 : 2;
   Q35_CHECK_ARG(A && B && C && M > 0 && N > 0 && K > 0 && tile < kPlanTiles);
   if (tile < 0) plan(M, N, K, kind, &tile, &splits);
   const bool ks = tile >= kTiles;
   Q35_CHECK_ARG(splits >= 1 && splits <= kMaxSplits);
-  Q35_CHECK_ARG(ks || kStaged[tile] || kind == KIND_BF16 || kind == KIND_I32);
+  Q35_CHECK_ARG(ks || kStaged[tile] || kind_direct(kind));
   Q35_CHECK_ARG(q35_aligned16(A) && q35_aligned16(B) && ((long long)K * es) % kRB == 0);
   Q35_CHECK_ARG((kind != KIND_DEQ && kind != KIND_DEQ_SWIGLU) || (s_x && s_w));
   // 32-bit byte offsets of every operand row
@@ -774,6 +800,8 @@ int gemm_run(const void* A, const void* B, void* C, int M, int N, int K, int kin
     case KIND_SWIGLU: return launch_tile<KIND_SWIGLU>(tile, a, stream);
     case KIND_I32: return launch_tile<KIND_I32>(tile, a, stream);
     case KIND_DEQ: return launch_tile<KIND_DEQ>(tile, a, stream);
+    case KIND_BIAS: return launch_tile<KIND_BIAS>(tile, a, stream);
+    case KIND_BIAS_GELU: return launch_tile<KIND_BIAS_GELU>(tile, a, stream);
     default: return launch_tile<KIND_DEQ_SWIGLU>(tile, a, stream);
   }
 }
@@ -806,8 +834,19 @@ long long q35_gemm_workspace(int M, int N, int K, int kind, int tile, int splits
 int q35_gemm(const void* A, const void* B, void* C, int M, int N, int K, int kind, const void* s_x,
              const void* s_w, int tile, int splits, void* workspace, long long workspace_bytes,
              hipStream_t stream) {
+  Q35_CHECK_ARG(kind >= 0 && kind < kNumKinds);
   return gemm_run(A, B, C, M, N, K, kind, (const float*)s_x, (const float*)s_w, tile, splits,
                   workspace, workspace_bytes, stream);
+}
+
+// C[M, N] = bf16(A . B^T + bias), or with gelu bf16(GELU_tanh(A . B^T + bias)),
+// bias [N] bf16, the sum and the GELU on the fp32 accumulators. K % 64 == 0; A
+// and B 16-byte aligned; the default plan, no workspace.
+int q35_gemm_bias(const void* A, const void* B, const void* bias, void* C, int M, int N, int K, int gelu,
+                  hipStream_t stream) {
+  Q35_CHECK_ARG(bias != nullptr);
+  return gemm_run(A, B, C, M, N, K, gelu ? KIND_BIAS_GELU : KIND_BIAS, nullptr, (const float*)bias, -1, 1, nullptr,
+                  0, stream);
 }
 
 }  // extern "C"

@@ -28,8 +28,8 @@
 
 namespace {
 
-enum { KIND_BF16 = 0, KIND_SWIGLU = 1, KIND_I32 = 2, KIND_DEQ = 3, KIND_DEQ_SWIGLU = 4 };
-constexpr int kNumKinds = 5;
+enum { KIND_BF16 = 0, KIND_SWIGLU = 1, KIND_I32 = 2, KIND_DEQ = 3, KIND_DEQ_SWIGLU = 4, KIND_BIAS = 5, KIND_BIAS_GELU = 6 };
+constexpr int kNumKinds = 5;  // kinds of q35_gemm; the bias kinds have their own entry
 
 struct GemmArgs {
   const uint8_t* A;  // [M, K]
@@ -37,7 +37,7 @@ struct GemmArgs {
   void* C;           // [M, N] bf16 or int32
   int M, N, K;       // K in elements
   const float* s_x;  // int8 kinds 3, 4: per-row scales of A
-  const float* s_w;  // per-row scales of B
+  const float* s_w;  // per-row scales of B; bias kinds: the bf16 bias [N]
   unsigned* cnt;     // split-K arrival counters, one per tile
   uint8_t* part;     // split-K partial tiles
   int splits, kps;   // splits per tile, stages per split
@@ -46,8 +46,13 @@ struct GemmArgs {
 template <bool I8> struct GemmAcc { using T = q35_f32x16; using E = float; using Q = q35_f32x4; };
 template <> struct GemmAcc<true> { using T = q35_i32x16; using E = int; using Q = q35_i32x4; };
 
-constexpr bool kind_i8(int kind) { return kind >= KIND_I32; }
+constexpr bool kind_i8(int kind) { return kind >= KIND_I32 && kind <= KIND_DEQ_SWIGLU; }
+constexpr bool kind_bias(int kind) { return kind == KIND_BIAS || kind == KIND_BIAS_GELU; }
+// bf16 or int32 values straight from the accumulators
+constexpr bool kind_direct(int kind) { return kind == KIND_BF16 || kind == KIND_I32 || kind_bias(kind); }
 constexpr bool kind_swiglu(int kind) { return kind == KIND_SWIGLU || kind == KIND_DEQ_SWIGLU; }
+
+Q35_DEV float bias_at(const GemmArgs& a, int n) { return bf2f(reinterpret_cast<const uint16_t*>(a.s_w)[n]); }
 
 // Slot of 16-byte chunk c of tile row r in the swizzled LDS image.
 template <int RB>
@@ -233,6 +238,8 @@ __global__ __launch_bounds__(W * 64) void gemm_ksplit(const GemmArgs a) {
           for (int e = 0; e < 4; ++e) {
             if constexpr (I8) v[g][e] = (float)s[g][e] * sx * a.s_w[g * a.N + min(n + e, a.N - 1)];
             else v[g][e] = s[g][e];
+            if constexpr (kind_bias(KIND)) v[g][e] += bias_at(a, min(n + e, a.N - 1));
+            if constexpr (KIND == KIND_BIAS_GELU) v[g][e] = gelu_tanh_fast(v[g][e]);
           }
         if constexpr (SWIGLU) {
 #pragma unroll

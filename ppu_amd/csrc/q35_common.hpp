@@ -70,6 +70,12 @@ Q35_DEV float silu_f(float x) { return x / (1.0f + expf(-x)); }
 // immediately: the fp32 difference moves that rounding only for values within
 // a few ulp of a bf16 rounding boundary.
 Q35_DEV float silu_fast(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
+// GELU with the tanh approximation, x/2 (1 + tanh u) = x / (1 + e^{-2u}), u =
+// sqrt(2/pi) (x + 0.044715 x^3), from the same hardware functions.
+Q35_DEV float gelu_tanh_fast(float x) {
+  const float u2 = x * fmaf(0.07135481282f, x * x, 1.5957691216f);
+  return x * __builtin_amdgcn_rcpf(1.0f + __expf(-u2));
+}
 Q35_DEV float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
 // ---------------------------------------------------------------- DPP moves
 template <int CTRL>

@@ -591,6 +591,25 @@ def gemm_bf16(x: torch.Tensor, weight: torch.Tensor, *, swiglu: bool = False,
 
 
 @_device_checked
+def gemm_bias(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, *,
+              gelu: bool = False) -> torch.Tensor:
+    """``F.linear(x, W, bias)`` on the hand-written matrix-core GEMM (bf16,
+    the bias added to the fp32 accumulator), or with ``gelu`` its
+    tanh-approximated GELU in the same epilogue: the vision tower's linears.
+    No counterpart in the reference's kernel API. K must be a multiple of 64."""
+
+    x2, n = _gemm_operands(x, weight, _BF16, False)
+    if bias.shape != (n,) or not bias.is_contiguous():
+        raise ValueError(f"bias must be a contiguous [{n}] tensor")
+    _need_bf16(bias)
+    y = torch.empty((*x.shape[:-1], n), device=x.device, dtype=_BF16)
+    if x2.shape[0]:
+        _lib.call("q35_gemm_bias", x2.data_ptr(), weight.data_ptr(), bias.data_ptr(), y.data_ptr(),
+                  x2.shape[0], n, x2.shape[1], int(gelu), _stream(x))
+    return y
+
+
+@_device_checked
 def ppu_swiglu_gemv(
     x: torch.Tensor,
     packed_weight: torch.Tensor,

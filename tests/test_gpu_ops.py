@@ -1356,6 +1356,38 @@ def test_gemm_ksplit_bf16(gpu, m, n, k):
     assert torch.equal(K.gemm_into(xd, wd, y2, K.GEMM_BF16), y[:m])
 
 
+# ring tiles (128x128 and 128-row direct, 256 wide) besides the K-splitting ones
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("m,n,k", _KS_SHAPES[1:12:2] + [(784, 4352, 1152), (785, 3450, 320), (1600, 4304, 192),
+                                                        (4100, 1154, 128), (4096, 4608, 256)])
+def test_gemm_bias(gpu, m, n, k, gelu):
+    """Linear with a bias, and with the tanh GELU, in the GEMM's epilogue: fp64
+    of the same operands, no write past the output, no larger an error than
+    the library's linear."""
+    from ppu_amd import kernels as K, _lib
+
+    g = gen(KERNEL_SEED + 99)
+    x, w = randn(g, m, k).to(gpu), randn(g, n, k, scale=2 * k**-0.5).to(gpu)
+    b = randn(g, n, scale=2.0).to(gpu)
+    y = torch.full((m + 1, n), 7.0, dtype=BF, device=gpu)
+    _lib.call("q35_gemm_bias", x.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), m, n, k, int(gelu),
+              _lib.stream(x.device))
+    ref = x.double() @ w.double().t() + b.double()
+    # the fp32 sum of k + 1 terms; GELU's slope is at most 1.13, its exponential
+    # and reciprocal are right to 2^-15; one bf16 rounding
+    err = (k + 1) * 2.0**-24 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+    lib = torch.nn.functional.linear(x, w, b)
+    if gelu:
+        ref = torch.nn.functional.gelu(ref, approximate="tanh")
+        err = 1.13 * err + 2.0**-15 * ref.abs()
+        lib = torch._addmm_activation(b, x, w.t(), use_gelu=True)
+    bound = ref.abs() * 2.0**-8 + err + 1e-30
+    assert bool(((y[:m].double() - ref).abs() <= bound).all())
+    assert bool((y[m] == 7.0).all())
+    assert (y[:m].double() - ref).norm() <= 1.01 * (lib.double() - ref).norm()
+    assert torch.equal(K.gemm_bias(x, w, b, gelu=gelu), y[:m])
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 6144, 2048), (64, 6144, 128), (90, 6100, 2048), (128, 6144, 256),
                                    (150, 6144, 2048), (256, 6140, 512), (5, 24, 192)])
 def test_gemm_ksplit_swiglu(gpu, m, n, k):
