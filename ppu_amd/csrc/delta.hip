@@ -663,10 +663,25 @@ struct ConvIn {
   uint16_t* state;    // [B, 3*H*D, 4]
 };
 
+// 4 values of one LDS column per lane (rows of 4 tokens): lane i of 16 gives
+// the address of 4 values of row i / 4 and receives column i.
+Q35_DEV uint2 dc_read_tr16(const uint16_t* p) {
+  typedef short q35_i16x4c __attribute__((ext_vector_type(4)));
+  const q35_i16x4c v =
+      __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) q35_i16x4c*)(p));
+  return __builtin_bit_cast(uint2, v);
+}
+
+// Bound by each workgroup's serial chain (conv, factors, A, T, W), so what
+// counts is waves per SIMD: 8 waves and 79 KiB of LDS (T takes Q's place, the
+// transpose tiles A's) put two workgroups on a CU, where 4 waves and 125 KiB
+// left one wave per SIMD. 16 heads: 40 -> 26 us at 2003 tokens (512 workgroups),
+// 18.8 -> 16 at 340 (96).
 // PF32: A_log and dt_bias are fp32 (else bf16); a template parameter, since a
 // run-time branch between two load forms makes the compiler wait for each.
+constexpr int kPrepThreads = 512;
 template <bool PF32, bool CONV>
-__global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restrict__ qkv,
+__global__ __launch_bounds__(kPrepThreads, 4) void delta_chunk_prep(const uint16_t* __restrict__ qkv,
                                                         int qkv_stride,
                                                         const uint16_t* __restrict__ packed,
                                                         int packed_stride, const void* a_log,
@@ -681,86 +696,98 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
   const int col = lane & 15, g4 = lane >> 4;
   const size_t bhc = ((size_t)b * H + h) * nC + c;
   float* wsb = ws + bhc * kChunkFloats;
-  __shared__ alignas(16) uint16_t Qr[kChunk * kRS];  // raw q, k, v rows (bf16)
+  // raw q, k, v rows (bf16); T = (I + A)^{-1} (lower) takes q's place
+  __shared__ alignas(16) uint16_t Qr[kChunk * kRS];
   __shared__ alignas(16) uint16_t Kr[kChunk * kRS];
   __shared__ alignas(16) uint16_t Vr[kChunk * kRS];
-  __shared__ alignas(16) float Am[kChunk * kAS];     // A (strictly lower)
-  __shared__ alignas(16) float Tm[kChunk * kAS];     // T = (I + A)^{-1} (lower)
-  __shared__ alignas(16) float Xs[4][kChunk * kXS];  // per-wave transpose tiles
+  // A (strictly lower), then per-wave transpose tiles of 320 floats; W's
+  // transpose tiles (864 floats per wave) take both places
+  __shared__ alignas(16) float AX[kChunk * kAS + 8 * 320];
   __shared__ alignas(16) float G_s[kChunk], b_s[kChunk], qinv_s[kChunk], kinv_s[kChunk], wsc_s[kChunk];
+  static_assert(sizeof(Qr) >= kChunk * kAS * 4, "T fits q's place");
+  static_assert(8 * 864 * 4 <= sizeof(AX) && 16 * kXS <= 864, "W's transpose tiles fit");
+  float* const Tm = reinterpret_cast<float*>(Qr);
+  float* const Am = AX;
+  float* const xs = AX + kChunk * kAS + wid * 320;
 
   // The token's gate inputs and the head's parameters, requested first (with
   // CONV they are then in flight during the conv below).
-  const int ti = tid >> 2;
+  const int ti = tid >> 3;
   const int tcg = min(c * kChunk + ti, L - 1);
   const uint16_t* prow0 = packed + ((size_t)b * L + tcg) * packed_stride;
   const float a_raw = bf2f(prow0[a_off + h]), b_raw = bf2f(prow0[b_off + h]);
   const float alog = ld_param(a_log, h, PF32), dtb = ld_param(dt_bias, h, PF32);
   if (CONV) {
     // 0. the conv of this chunk and head into Qr / Kr / Vr. Thread items are
-    //    (8-channel group g of q, k or v; 4 tokens), 768 of them (48 groups x
+    //    (4-channel group g of q, k or v; 4 tokens), 1536 of them (96 groups x
     //    16 token blocks), three per thread, each with its 7 input rows (4 + 3
-    //    before; rows before token 0 are zero) and 4 x 8 taps; every load of
+    //    before; rows before token 0 are zero) and 4 x 4 taps; every load of
     //    the three items is issued before any is used. The bf16 rounding of
     //    the conv sums takes one conversion per pair of values.
     {
       constexpr int NI = 3;
-      uint4 raw[NI][7], wr[NI][4];
+      uint2 raw[NI][7];
+      uint4 wr[NI][2];
 #pragma unroll
       for (int it = 0; it < NI; ++it) {
-        const int item = tid + 256 * it;
-        const int g = item % 48, t0 = (item / 48) * 4;
-        const int ch = (g >> 4) * H * kD + h * kD + (g & 15) * 8;  // conv channel of the group
+        const int item = tid + kPrepThreads * it;
+        const int g = item % 96, t0 = (item / 96) * 4;
+        const int ch = (g >> 5) * H * kD + h * kD + (g & 31) * 4;  // conv channel of the group
 #pragma unroll
         for (int r = 0; r < 7; ++r) {
           const int tr = min(max(c * kChunk + t0 - 3 + r, 0), L - 1);
-          raw[it][r] = *reinterpret_cast<const uint4*>(qkv + ((size_t)b * L + tr) * qkv_stride + ch);
+          raw[it][r] = *reinterpret_cast<const uint2*>(qkv + ((size_t)b * L + tr) * qkv_stride + ch);
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) wr[it][q] = *reinterpret_cast<const uint4*>(conv.w + (size_t)ch * 4 + q * 8);
+        for (int q = 0; q < 2; ++q) wr[it][q] = *reinterpret_cast<const uint4*>(conv.w + (size_t)ch * 4 + q * 8);
       }
 #pragma unroll
       for (int it = 0; it < NI; ++it) {
-        const int item = tid + 256 * it;
-        const int g = item % 48, t0 = (item / 48) * 4;
-        const int arr = g >> 4, d = (g & 15) * 8;
+        const int item = tid + kPrepThreads * it;
+        const int g = item % 96, t0 = (item / 96) * 4;
+        const int arr = g >> 5, d = (g & 31) * 4;
         const int ch = arr * H * kD + h * kD + d;
         uint16_t* dst = arr == 0 ? Qr : (arr == 1 ? Kr : Vr);
-        float wt[8][4];
+        float wt[4][4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < 2; ++q) {
           float f[8];
           unpack8(wr[it][q], f);
 #pragma unroll
           for (int e = 0; e < 8; ++e) wt[2 * q + e / 4][e % 4] = f[e];
         }
-        float xr[7][8];
+        float xr[7][4];
 #pragma unroll
         for (int r = 0; r < 7; ++r) {
           const bool before = c * kChunk + t0 - 3 + r < 0;
-          unpack8(before ? make_uint4(0u, 0u, 0u, 0u) : raw[it][r], xr[r]);
+          const uint2 x = before ? make_uint2(0u, 0u) : raw[it][r];
+          xr[r][0] = bf_lo(x.x);
+          xr[r][1] = bf_hi(x.x);
+          xr[r][2] = bf_lo(x.y);
+          xr[r][3] = bf_hi(x.y);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int t = c * kChunk + t0 + j;
-          float acc[8], o[8];
+          float acc[4], o[4];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
+          for (int e = 0; e < 4; ++e) {
             acc[e] = 0.f;
 #pragma unroll
             for (int tap = 0; tap < 4; ++tap) acc[e] = fmaf(xr[j + tap][e], wt[e][tap], acc[e]);
           }
 #pragma unroll
-          for (int p2 = 0; p2 < 4; ++p2) {
+          for (int p2 = 0; p2 < 2; ++p2) {
             const uint32_t hb = pack_bf2(acc[2 * p2], acc[2 * p2 + 1]);
             o[2 * p2] = silu_fast(bf_lo(hb));
             o[2 * p2 + 1] = silu_fast(bf_hi(hb));
           }
-          *reinterpret_cast<uint4*>(dst + (t0 + j) * kRS + d) = pack8(o);  // the conv output is bf16
+          // the conv output is bf16
+          *reinterpret_cast<uint2*>(dst + (t0 + j) * kRS + d) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
           const int pos = t - (L - 4);
           if (t < L && pos >= 0) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
+            for (int e = 0; e < 4; ++e)
               conv.state[((size_t)b * 3 * H * kD + ch + e) * 4 + pos] = (uint16_t)f2bf(xr[j + 3][e]);
           }
         }
@@ -769,24 +796,23 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
     __syncthreads();
   }
 
-  // 1. per token (4 threads, 32 dims each): q_inv, k_inv = rsqrt(sum of
-  //    squares + 1e-6) over the head (quad sum), g = -e^{A_log} softplus(a +
-  //    dt_bias), beta = sigmoid(b) [reference kernels.py:713-765]. The raw
-  //    rows of tokens past L become zeros; the q rows are also the output
-  //    kernel's A operand (row tile i/16, k step = the thread's quarter,
-  //    lane (i%16) + 16u for its 8-dim group u).
+  // 1. per token (8 threads, 16 dims each): q_inv, k_inv = rsqrt(sum of
+  //    squares + 1e-6) over the head (sum of 8 lanes), g = -e^{A_log}
+  //    softplus(a + dt_bias), beta = sigmoid(b) [reference
+  //    kernels.py:713-765]. The raw rows of tokens past L become zeros; the q
+  //    rows are also the output kernel's A operand (row tile i/16, k step =
+  //    the thread pair's 32 dims, lane (i%16) + 16u for its 8-dim group u).
   {
-    const int i = tid >> 2, qq = tid & 3;
+    const int i = tid >> 3, qq = tid & 7;
     const int t = c * kChunk + i;
     const bool live = t < L;
-    uint4 rq[4], rk[4], rv[4];
+    uint4 rq[2], rk[2], rv[2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int d = qq * 32 + u * 8;
+    for (int u = 0; u < 2; ++u) {
+      const int d = qq * 16 + u * 8;
       if (CONV) {
         rq[u] = *reinterpret_cast<const uint4*>(&Qr[i * kRS + d]);
         rk[u] = *reinterpret_cast<const uint4*>(&Kr[i * kRS + d]);
-        rv[u] = *reinterpret_cast<const uint4*>(&Vr[i * kRS + d]);
       } else {
         const uint16_t* row = qkv + ((size_t)b * L + min(t, L - 1)) * qkv_stride;
         rq[u] = *reinterpret_cast<const uint4*>(row + h * kD + d);
@@ -796,7 +822,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
     }
     float qs = 0.f, ks = 0.f;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < 2; ++u) {
       float fq[8], fk[8];
       unpack8(rq[u], fq);
       unpack8(rk[u], fk);
@@ -806,26 +832,28 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
         ks += fk[e] * fk[e];
       }
     }
-    qs += __shfl_xor(qs, 1, 64);
-    ks += __shfl_xor(ks, 1, 64);
-    qs += __shfl_xor(qs, 2, 64);
-    ks += __shfl_xor(ks, 2, 64);
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      qs += __shfl_xor(qs, o, 64);
+      ks += __shfl_xor(ks, o, 64);
+    }
     if (!live) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) rq[u] = rk[u] = rv[u] = make_uint4(0u, 0u, 0u, 0u);
+      for (int u = 0; u < 2; ++u) rq[u] = rk[u] = rv[u] = make_uint4(0u, 0u, 0u, 0u);
     }
     if (!CONV || !live) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int d = qq * 32 + u * 8;
+      for (int u = 0; u < 2; ++u) {
+        const int d = qq * 16 + u * 8;
         *reinterpret_cast<uint4*>(&Qr[i * kRS + d]) = rq[u];
         *reinterpret_cast<uint4*>(&Kr[i * kRS + d]) = rk[u];
         *reinterpret_cast<uint4*>(&Vr[i * kRS + d]) = rv[u];
       }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      *reinterpret_cast<uint4*>(wsb + kOffQ + (((i >> 4) * 4 + qq) * 64 + (i & 15) + 16 * u) * 4) = rq[u];
+    for (int u = 0; u < 2; ++u)
+      *reinterpret_cast<uint4*>(wsb + kOffQ + (((i >> 4) * 4 + (qq >> 1)) * 64 + (i & 15) + 16 * (2 * (qq & 1) + u)) * 4) =
+          rq[u];
     if (qq == 0) {
       qinv_s[i] = rsqrt_cr(qs + 1e-6f);
       kinv_s[i] = rsqrt_cr(ks + 1e-6f);
@@ -852,50 +880,57 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
     wsb[kOffSc + lane] = gam * qinv_s[lane] * kQScale;
     if (lane == 0) gc_out[bhc] = expf(glast);
   }
-  __syncthreads();
 
   // 3. A (into LDS) and P (split, to the workspace) on the lower block
   //    triangle. P is exported by (row tile rt, t step s) groups of two tiles
   //    (jt = 2s, 2s + 1; a tile above the diagonal is zero), each group on one
-  //    wave, so its transpose goes through the wave's own tile: wave 0 takes
-  //    (3, 0) and (0, 0), wave 1 (3, 1) and (2, 1), wave 2 (1, 0), wave 3
-  //    (2, 0): 3/3/2/2 tiles. Operands are raw rows of 16 bytes.
+  //    wave, so its transpose goes through the wave's own tile: waves 0 to 5
+  //    take (3, 0), (3, 1), (2, 0), (1, 0), (0, 0), (2, 1). Operands are raw
+  //    rows of 16 bytes; the products need no decay, so they run beside 2.
   {
-    const unsigned groups = wid == 0 ? 0x0300u : (wid == 1 ? 0x0607u : (wid == 2 ? 0x01u : 0x02u));
-    const int ng = wid < 2 ? 2 : 1;
-    float* xs = Xs[wid];
-    for (int n = 0; n < ng; ++n) {
-      const int gi = (groups >> (8 * n)) & 0xff;
-      const int rt = gi & 3, s = gi >> 2;
+    const int rt = (0x201233 >> (4 * wid)) & 3, s = (0x22 >> wid) & 1;
+    q35_f32x4 kk[2], qk[2];
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      const int jt = 2 * s + jj;
+      kk[jj] = qk[jj] = q35_f32x4{0.f, 0.f, 0.f, 0.f};
+      if (wid < 6 && jt <= rt) {
+        const uint16_t* ki = &Kr[(16 * rt + col) * kRS + 8 * g4];
+        const uint16_t* kj = &Kr[(16 * jt + col) * kRS + 8 * g4];
+        const uint16_t* qi = &Qr[(16 * rt + col) * kRS + 8 * g4];
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+          const uint4 x = *reinterpret_cast<const uint4*>(ki + 32 * st);
+          const uint4 y = *reinterpret_cast<const uint4*>(kj + 32 * st);
+          const uint4 z = *reinterpret_cast<const uint4*>(qi + 32 * st);
+          kk[jj] = mfma_bf(x, y, kk[jj]);  // (k k^T)[i][j]
+          qk[jj] = mfma_bf(z, y, qk[jj]);  // (q k^T)[i][j]
+        }
+      }
+    }
+    __syncthreads();  // G_s, wsc_s; the last read of q
+    if (wid < 6) {
+      float4 p0, p1;
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
         const int jt = 2 * s + jj;
-        q35_f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
-        if (jt <= rt) {
-          const uint16_t* ki = &Kr[(16 * rt + col) * kRS + 8 * g4];
-          const uint16_t* kj = &Kr[(16 * jt + col) * kRS + 8 * g4];
-          const uint16_t* qi = &Qr[(16 * rt + col) * kRS + 8 * g4];
-#pragma unroll
-          for (int st = 0; st < 4; ++st) {
-            const uint4 x = *reinterpret_cast<const uint4*>(ki + 32 * st);
-            const uint4 y = *reinterpret_cast<const uint4*>(kj + 32 * st);
-            const uint4 z = *reinterpret_cast<const uint4*>(qi + 32 * st);
-            kk = mfma_bf(x, y, kk);  // (k k^T)[i][j]
-            qk = mfma_bf(z, y, qk);  // (q k^T)[i][j]
-          }
-        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int i = 16 * rt + 4 * g4 + e, j = 16 * jt + col;
           const float dec = j <= i ? expf(G_s[i] - G_s[j]) : 0.f;
-          if (jt <= rt) Am[i * kAS + j] = j < i ? b_s[i] * (kinv_s[i] * kinv_s[j]) * dec * kk[e] : 0.f;
-          xs[(4 * g4 + e) * kXS + 16 * jj + col] = qinv_s[i] * kQScale * kinv_s[j] * dec * qk[e];
+          if (jt <= rt) Am[i * kAS + j] = j < i ? b_s[i] * (kinv_s[i] * kinv_s[j]) * dec * kk[jj][e] : 0.f;
+          xs[(4 * g4 + e) * 20 + col] = qinv_s[i] * kQScale * kinv_s[j] * dec * qk[jj][e];
+        }
+        // the tile as its half of the A operand (row 16 rt + l%16, columns 32 s
+        // + 8(l/16) .. +7); the wave's own LDS accesses keep their order
+        const float* pr = &xs[col * 20 + 8 * (g4 & 1)];
+        const float4 x0 = *reinterpret_cast<const float4*>(pr), x1 = *reinterpret_cast<const float4*>(pr + 4);
+        if (jj == 0 || g4 >= 2) {
+          p0 = x0;
+          p1 = x1;
         }
       }
-      // the group as the A operand (row 16 rt + l%16, columns 32 s + 8(l/16)
-      // .. +7); the wave's own LDS stores complete before its later reads
-      const float* pr = &xs[col * kXS + 8 * g4];
-      const Split8 sp = split8(*reinterpret_cast<const float4*>(pr), *reinterpret_cast<const float4*>(pr + 4));
+      const Split8 sp = split8(p0, p1);
       uint4* dp = reinterpret_cast<uint4*>(wsb + kOffP) + (rt * 2 + s) * 128 + lane;
       dp[0] = sp.hi;
       dp[64] = sp.lo;
@@ -907,7 +942,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
   //    T_II = (I + A_II)^{-1} by forward substitution (wave I, lane = column),
   //    then T_IJ = -T_II sum_{K=J}^{I-1} A_IK T_KJ level by level (I - J =
   //    1, 2, 3) as 16 x 16 x 16 fp32 MFMA products, one block per wave.
-  {
+  if (wid < 4) {
     const int I = wid, j = lane & 15;
     float t[16];
 #pragma unroll
@@ -926,6 +961,22 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
       for (int i = 0; i < 16; ++i) Tm[(16 * I + i) * kAS + 16 * I + j] = t[i];
     }
   }
+  // the wave's k and v columns of step 5 (8 consecutive tokens of one dim; k's
+  // also the kT operand of the scan), tiles dt = 2 (wid % 4) + dd
+  uint4 kop[2][2], vop[2][2];
+  const int dt0 = 2 * (wid & 3), half = wid >> 2;
+#pragma unroll
+  for (int dd = 0; dd < 2; ++dd)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int at = (32 * s + 8 * g4 + (col >> 2)) * kRS + 16 * (dt0 + dd) + 4 * (col & 3);
+      const uint2 k0 = dc_read_tr16(&Kr[at]), k1 = dc_read_tr16(&Kr[at + 4 * kRS]);
+      const uint2 v0 = dc_read_tr16(&Vr[at]), v1 = dc_read_tr16(&Vr[at + 4 * kRS]);
+      kop[dd][s] = make_uint4(k0.x, k0.y, k1.x, k1.y);
+      vop[dd][s] = make_uint4(v0.x, v0.y, v1.x, v1.y);
+      if (s == half)
+        *reinterpret_cast<uint4*>(wsb + kOffKT + (((dt0 + dd) * 2 + s) * 64 + lane) * 4) = kop[dd][s];
+    }
   __syncthreads();
   // C += A B for 16 x 16 tiles in LDS (A row stride kAS, B row stride sb).
   auto mm16 = [&](const float* at, const float* bt, int sb, q35_f32x4 c) {
@@ -938,7 +989,6 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
       const int J = wid, I = wid + d;
       q35_f32x4 x = {0.f, 0.f, 0.f, 0.f};
       for (int K = J; K < I; ++K) x = mm16(&Am[16 * I * kAS + 16 * K], &Tm[16 * K * kAS + 16 * J], kAS, x);
-      float* xs = Xs[wid];
 #pragma unroll
       for (int e = 0; e < 4; ++e) xs[(4 * g4 + e) * 17 + col] = x[e];
       // the wave's own LDS stores complete before its later reads (in-order LDS)
@@ -950,38 +1000,21 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
   }
 
   // 5. W = (T diag(beta gamma k_inv)) k and U0 = (T diag(beta)) v for the
-  //    wave's two dim (v) tiles dt = 2 wid + dd and every row tile: the T rows
-  //    are split, the k / v columns (8 consecutive tokens of one dim; the kT
-  //    operand of the scan) are exact. T is lower triangular: row tile rt
-  //    needs the t steps s <= rt/2, and the lane's 8 columns of block
-  //    2s + (l/16)/2 are zero when that block is above the diagonal.
+  //    wave's two dim (v) tiles and two row tiles, 3 and 0 on waves 0 to 3, 2
+  //    and 1 on waves 4 to 7: the T rows are split, the k / v columns are
+  //    exact. T is lower triangular: row tile rt needs the t steps s <= rt/2,
+  //    and the lane's 8 columns of block 2s + (l/16)/2 are zero when that
+  //    block is above the diagonal.
   {
-    uint4 kop[2][2], vop[2][2];
+    float* xw = AX + wid * 864;  // W rows of one row tile, columns 16 dt0 .. +31
 #pragma unroll
-    for (int dd = 0; dd < 2; ++dd)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int dim = 16 * (2 * wid + dd) + col;
-        const uint16_t* kc = &Kr[(32 * s + 8 * g4) * kRS + dim];
-        const uint16_t* vc = &Vr[(32 * s + 8 * g4) * kRS + dim];
-        uint32_t kw[4], vw[4];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-          kw[p] = (uint32_t)kc[2 * p * kRS] | ((uint32_t)kc[(2 * p + 1) * kRS] << 16);
-          vw[p] = (uint32_t)vc[2 * p * kRS] | ((uint32_t)vc[(2 * p + 1) * kRS] << 16);
-        }
-        kop[dd][s] = make_uint4(kw[0], kw[1], kw[2], kw[3]);
-        vop[dd][s] = make_uint4(vw[0], vw[1], vw[2], vw[3]);
-        *reinterpret_cast<uint4*>(wsb + kOffKT + (((2 * wid + dd) * 2 + s) * 64 + lane) * 4) = kop[dd][s];
-      }
-    float* xw = Xs[wid];  // W rows 0..63, columns 32 wid .. +31
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
+    for (int r = 0; r < 2; ++r) {
+      const int rt = r == 0 ? 3 - half : half;
       q35_f32x4 w[2], u[2];
 #pragma unroll
       for (int dd = 0; dd < 2; ++dd) w[dd] = u[dd] = q35_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s <= rt / 2; ++s) {
+      for (int s = 0; s < 2 - r; ++s) {
         const int j0 = 32 * s + 8 * g4;
         float4 t0 = make_float4(0.f, 0.f, 0.f, 0.f), t1 = t0;
         if (2 * s + (g4 >> 1) <= rt) {
@@ -1010,18 +1043,15 @@ __global__ __launch_bounds__(256) void delta_chunk_prep(const uint16_t* __restri
       }
 #pragma unroll
       for (int dd = 0; dd < 2; ++dd) {
-        *reinterpret_cast<float4*>(wsb + kOffU0 + ((rt * 8 + 2 * wid + dd) * 64 + lane) * 4) =
+        *reinterpret_cast<float4*>(wsb + kOffU0 + ((rt * 8 + dt0 + dd) * 64 + lane) * 4) =
             make_float4(u[dd][0], u[dd][1], u[dd][2], u[dd][3]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) xw[(16 * rt + 4 * g4 + e) * kXS + 16 * dd + col] = w[dd][e];
+        for (int e = 0; e < 4; ++e) xw[(4 * g4 + e) * kXS + 16 * dd + col] = w[dd][e];
       }
-    }
-    // W as the scan's A operand: row 16 rt + l%16, dims 32 wid + 8(l/16) .. +7
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      const float* wr = &xw[(16 * rt + col) * kXS + 8 * g4];
+      // W as the scan's A operand: row 16 rt + l%16, dims 16 dt0 + 8(l/16) .. +7
+      const float* wr = &xw[col * kXS + 8 * g4];
       const Split8 sp = split8(*reinterpret_cast<const float4*>(wr), *reinterpret_cast<const float4*>(wr + 4));
-      uint4* dp = reinterpret_cast<uint4*>(wsb + kOffW) + (rt * 4 + wid) * 128 + lane;
+      uint4* dp = reinterpret_cast<uint4*>(wsb + kOffW) + (rt * 4 + (wid & 3)) * 128 + lane;
       dp[0] = sp.hi;
       dp[64] = sp.lo;
     }
@@ -1520,7 +1550,7 @@ int delta_prefill(const void* qkv, int qkv_stride, const void* packed, int packe
   float* snap = gc + (((size_t)B * H * nC + 3) & ~(size_t)3);
   const ConvIn cv = conv ? *conv : ConvIn{nullptr, nullptr};
 #define PREP(PF, CV)                                                                              \
-  delta_chunk_prep<PF, CV><<<dim3(nC, H, B), 256, 0, stream>>>(                                   \
+  delta_chunk_prep<PF, CV><<<dim3(nC, H, B), kPrepThreads, 0, stream>>>(                          \
       (const uint16_t*)qkv, qkv_stride, (const uint16_t*)packed, packed_stride, a_log, dt_bias,   \
       params_f32, 4 * H * D, 4 * H * D + H, chunk_ws, gc, L, H, nC, cv)
   if (params_f32) {
