@@ -320,6 +320,35 @@ def test_lm_head_argmax(gpu, v, k):
         pytest.fail(f"argmax {int(got)} vs {int(exp)}: logits {a} vs {b}")
 
 
+@pytest.mark.parametrize("vocab", [1, 50001, 248320])
+def test_lm_head_logits_of_one_position(gpu, vocab):
+    """The language model head's module on one row runs the GEMV: fp64 of the
+    same operands; further rows, a bias or gradients keep the module's own."""
+    from ppu_amd import integration
+
+    g = gen(KERNEL_SEED + 41)
+    head = torch.nn.Linear(2048, vocab, bias=False, device=gpu, dtype=BF)
+    with torch.no_grad():
+        head.weight.copy_(randn(g, vocab, 2048, scale=0.02))
+    fast = integration._lm_head_fast(head)
+    x = randn(g, 1, 1, 2048).to(gpu)
+    assert fast(x) is NotImplemented  # the weight asks for gradients
+    with torch.no_grad():
+        y = fast(x)
+        assert y.shape == (1, 1, vocab) and y.dtype == BF
+        xd = x.reshape(-1).double()
+        for rows in range(0, vocab, 65536):
+            w = head.weight[rows : rows + 65536].double()
+            exp = w @ xd
+            # half a bf16 ulp of the result and the fp32 sum of 2048 terms
+            bound = exp.abs() * 2.0**-8 + 2048 * 2.0**-24 * (w.abs() @ xd.abs()) + 1e-30
+            assert bool(((y.reshape(-1)[rows : rows + 65536].double() - exp).abs() <= bound).all())
+        assert fast(x.expand(1, 2, 2048)) is NotImplemented
+        assert fast(x.float()) is NotImplemented
+        head.bias = torch.nn.Parameter(torch.zeros(vocab, device=gpu, dtype=BF))
+        assert fast(x) is NotImplemented
+
+
 def test_lm_head_ties(gpu):
     from ppu_amd import kernels as K
 
