@@ -34,6 +34,8 @@ from dataclasses import dataclass
 from typing import Any, Callable
 
 import torch
+from torch.autograd import forward_ad
+from torch.nn.modules import module as module_hooks
 from transformers.activations import GELUTanh
 from transformers.cache_utils import DynamicCache
 from transformers.models.qwen3_5 import modeling_qwen3_5 as qwen_impl
@@ -79,6 +81,16 @@ class FusionConfig:
 
 def _gpu_bf16(t: Any) -> bool:
     return isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.bfloat16
+
+
+def _values_only(*tensors: torch.Tensor) -> bool:
+    """Whether a product of these tensors may be taken from their memory alone:
+    no gradient, forward-mode tangent, autocast or function transform (vmap and
+    its like, whose tensors have no storage) asks for more, and no compiler is
+    tracing the call."""
+    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or forward_ad._current_level >= 0
+                or any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
+                or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
 
 
 def text_stack(model: torch.nn.Module) -> torch.nn.Module:
@@ -257,8 +269,7 @@ def _lm_head_fast(module):
         if (args or kwargs or not isinstance(x, torch.Tensor) or x.dim() == 0 or x.numel() != x.shape[-1]
                 or module.bias is not None or not (_gpu_bf16(x) and _gpu_bf16(w)) or x.device != w.device
                 or x.shape[-1] != w.shape[1] or not w.is_contiguous()
-                or (x.data_ptr() | w.data_ptr()) % 16 or torch.is_autocast_enabled()
-                or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+                or not _values_only(x, w) or (x.data_ptr() | w.data_ptr()) % 16):
             return NotImplemented
         return K.linear(x, w)
     return fast
@@ -690,9 +701,8 @@ def _bias_linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, gelu:
     call is 15 % less."""
     if (b is not None and x.dim() == 2 and x.shape[0] and _gpu_bf16(x) and _gpu_bf16(w) and _gpu_bf16(b)
             and w.device == x.device == b.device and w.shape[1] == x.shape[1] and w.shape[1] % 64 == 0
-            and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
-            and max(x.shape[0], w.shape[0]) * w.shape[1] < 1 << 30 and not torch.is_autocast_enabled()
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or b.requires_grad))):
+            and w.is_contiguous() and b.is_contiguous() and _values_only(x, w, b) and w.data_ptr() % 16 == 0
+            and max(x.shape[0], w.shape[0]) * w.shape[1] < 1 << 30):
         x = x.contiguous()
         if x.data_ptr() % 16 == 0:
             return K.gemm_bias(x, w, b, gelu=gelu)
@@ -703,9 +713,11 @@ def _bias_linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, gelu:
 
 def _bias_module(linear: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``linear(x)``; a plain ``nn.Linear`` without hooks goes straight to its
-    product, anything else (a wrapped or hooked module) is called."""
+    product, anything else (a wrapped module, or one with hooks of its own or
+    of every module, forward or backward) is called."""
     if (type(linear) is torch.nn.Linear and "forward" not in linear.__dict__
-            and not (linear._forward_hooks or linear._forward_pre_hooks)):
+            and not (linear._forward_hooks or linear._forward_pre_hooks or linear._backward_hooks
+                     or linear._backward_pre_hooks or module_hooks._has_any_global_hook())):
         return _bias_linear(x, linear.weight, linear.bias)
     return linear(x)
 
