@@ -21,15 +21,6 @@ Q35_DEV uint2 lds_read_tr16(const void* p) {
       __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) q35_i16x4*)(p));
   return __builtin_bit_cast(uint2, v);
 }
-// Lane l and lane l ^ 32: the larger of the two, their sum.
-Q35_DEV float half_max(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-Q35_DEV float half_sum(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 // 16-byte chunk c of a staged K or V row (32 chunks) sits at slot
 // c ^ fa_swz(row): the 16 rows of a K fragment read and the 4 rows x 4 chunks
 // of a transposed V read each fall on 16 distinct bank groups.

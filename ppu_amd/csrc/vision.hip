@@ -23,7 +23,7 @@
 // widths a lane-strided scalar form. The RoPE split runs one thread per four
 // rotation pairs (or one wave per (token, head) for other head dims). Builds
 // use -ffp-contract=off, so a*b+c is fused only where fmaf is written.
-#include "q35_common.hpp"
+#include "q35_tile.hpp"
 
 namespace {
 
@@ -349,34 +349,33 @@ __global__ __launch_bounds__(256) void vision_qkv_rope_vec(
 
 // ------------------------------------------------------ vision attention
 // Non-causal multi-head attention of the vision blocks on the matrix cores
-// (v_mfma_f32_16x16x32_bf16), one workgroup per (64 query rows, head), four
-// waves of 16 rows each; keys in blocks of 64 staged once in LDS for all four
-// waves (double buffered, the next block loaded into registers while the
-// current one is computed). Head dims D (D % 8 == 0, D <= 128) are zero-padded
-// to 32 QT (QT = ceil(D / 32)) in Q's registers and K's LDS rows; O has
-// OT = ceil(D / 16) tiles of 16 dims. Both are template parameters: a tile
+// (v_mfma_f32_32x32x16_bf16), one workgroup per (64 query rows, head): pairs of
+// waves with 32 rows each, every pair on its own 32 keys of a stage; the stages
+// are staged in LDS for all waves (double buffered, the next ones loaded into
+// registers while the current one is computed), and the pairs' partial results
+// merge through LDS at the end. The products are transposed, S^T = K Q^T and
+// O^T += V^T P^T: a lane holds one query row, so the softmax needs one exchange
+// between lanes l and l ^ 32, and the C layout of S^T, with the 16 keys of a k
+// step taken in the order {0-3, 8-11 | 4-7, 12-15}, already is the B operand of
+// O^T. Head dims D (D % 8 == 0, D <= 128) are zero-padded to KT = ceil(D / 16)
+// steps of S and DT = ceil(D / 32) tiles of O, both template parameters: a tile
 // count known only at run time put O behind branches, and the compiler then
-// copied the whole accumulator array at each one. Per block and
-// wave: S = Q K^T (4 x QT MFMAs), online softmax in fp32 (DPP row
-// reductions), P rounded to bf16 and written transposed to LDS, then O += P V
-// with P and V reaching the MFMA through the gfx950 transpose read
-// ds_read_b64_tr_b16 (the operand layouts and lane mapping of the causal
-// prefill kernel). Queries only see keys of their own image: image i holds
-// tokens [cu[i], cu[i+1]). Output rows go straight to [T, H*D], the layout the
-// output projection reads.
+// copied the whole accumulator array at each one. V reaches the MFMA through
+// the gfx950 transpose read ds_read_b64_tr_b16. Queries only see keys of their
+// own image: image i holds tokens [cu[i], cu[i+1]). Output rows go straight to
+// [T, H*D], the layout the output projection reads.
+//
+// Bound: the chain of stages of one workgroup per CU, of which the LDS reads
+// were the largest part with 16 rows per wave (every wave read 64 keys for
+// them, and P went through LDS). One 28 x 28 image, 16 heads of 72, 27 blocks:
+// the tower 2576 -> 2352 us, about 8 us per attention launch.
 typedef short q35_i16x4v __attribute__((ext_vector_type(4)));
 Q35_DEV uint2 va_read_tr16(const uint16_t* p) {
   const q35_i16x4v v =
       __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) q35_i16x4v*)(p));
   return __builtin_bit_cast(uint2, v);
 }
-Q35_DEV q35_f32x4 va_mfma(const uint4 a, const uint4 b, q35_f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(q35_bf16x8, a),
-                                                 __builtin_bit_cast(q35_bf16x8, b), c, 0, 0, 0);
-}
-
 typedef uint32_t va_u32x4 __attribute__((ext_vector_type(4)));
-constexpr int kVaKeys = 64;    // keys per block
 // K / V rows in LDS: 128 elements (16 chunks of 16 bytes) per key, chunk c of
 // row r stored at chunk c ^ va_swz(r % 16), a 4 x 4 transpose of the row's
 // low bits. The 16 rows of a K read (one chunk each) then sit on 16 distinct
@@ -385,7 +384,6 @@ constexpr int kVaKeys = 64;    // keys per block
 constexpr int kVaRS = 128;
 Q35_DEV int va_swz(int r15) { return ((r15 & 3) << 2) | ((r15 >> 2) & 3); }
 constexpr int kVaRows = 64;    // query rows per workgroup
-constexpr int kVaPt = 16 + 4;  // padded P^T row (16 query rows)
 
 // Image bounds [start, end) of token t (cu: n + 1 ascending offsets; none:
 // one image of T tokens).
@@ -402,106 +400,85 @@ Q35_DEV void va_segment(const int* cu, int n, int T, int t, int& s0, int& s1) {
   }
 }
 
-// One key block of one wave: S = Q K^T for its 16 rows x 64 keys, the online
+// One key block of one wave: S^T = K Q^T for 32 keys x its 32 rows, the online
 // softmax in base 2 (c = scale * log2(e) folded into one FMA per score; m is
-// kept in unscaled score units), bf16 P^T through the wave's LDS tile, then
-// O += P V. MASK: some key of the block lies outside a row's image (keys
-// outside get p = 0). lp holds this lane's partial row sums (the row sum is
-// one 16-lane reduction at the end).
-template <int QT, int OT, bool MASK>
+// kept in unscaled score units), O^T += V^T P^T with P rounded to bf16. A lane
+// holds one row (l32), half of its keys. MASK: some key of the block lies
+// outside a row's image (keys outside get p = 0). lp holds this lane's partial
+// row sum.
+template <int KT, int DT, bool MASK>
 Q35_DEV void va_block(const uint16_t* __restrict__ Ks, const uint16_t* __restrict__ Vs,
-                      uint16_t* __restrict__ pt, const uint4 (&qa)[QT], q35_f32x4 (&o)[OT],
-                      float (&m)[4], float (&lp)[4], int kb, const int (&s0)[4],
-                      const int (&s1)[4], float c, int col, int kg, int te, int tq) {
-  constexpr int RS = kVaRS;
-  const int gk = va_swz(col);  // K rows 16 st + col
-  q35_f32x4 s[4];
+                      const q35_u32x4 (&qa)[KT], q35_f32x16 (&o)[DT], float& m, float& lp, int kb,
+                      int s0, int s1, float c, int lane) {
+  const int l32 = lane & 31, kh = lane >> 5;
+  q35_f32x16 s;
 #pragma unroll
-  for (int st = 0; st < 4; ++st) {
-    s[st] = {0.f, 0.f, 0.f, 0.f};
-    const uint16_t* krow = Ks + (16 * st + col) * RS;
+  for (int r = 0; r < 16; ++r) s[r] = 0.f;
+  const uint16_t* krow = Ks + l32 * kVaRS;
 #pragma unroll
-    for (int t = 0; t < QT; ++t)
-      s[st] = va_mfma(qa[t], *reinterpret_cast<const uint4*>(krow + 8 * ((kg + 4 * t) ^ gk)), s[st]);
-  }
-  float corr[4], p[4][4];
-  bool moved = false;
+  for (int t = 0; t < KT; ++t)
+    s = mfma32(*reinterpret_cast<const q35_u32x4*>(krow + 8 * ((2 * t + kh) ^ va_swz(l32 & 15))), qa[t], s);
+  float mx = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float sv[4];
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-      sv[st] = s[st][i];
-      if (MASK) {
-        const int key = kb + 16 * st + col;
-        if (key < s0[i] || key >= s1[i]) sv[st] = -INFINITY;
-      }
+  for (int r = 0; r < 16; ++r) {
+    if (MASK) {
+      const int key = kb + 8 * (r >> 2) + 4 * kh + (r & 3);
+      if (key < s0 || key >= s1) s[r] = -INFINITY;
     }
-    const float m_new =
-        fmaxf(m[i], row16_max(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]))));
-    // A row with no key of its image so far keeps m = -inf: offset 0 then.
-    const float mc = (MASK && m_new == -INFINITY) ? 0.f : m_new * c;
-    moved |= m_new != m[i];
-    corr[i] = __builtin_amdgcn_exp2f(fmaf(m[i], c, -mc));
-    float ps = 0.f;
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-      p[st][i] = __builtin_amdgcn_exp2f(fmaf(sv[st], c, -mc));
-      ps += p[st][i];
-    }
-    lp[i] = fmaf(lp[i], corr[i], ps);
-    m[i] = m_new;
+    mx = fmaxf(mx, s[r]);
   }
-#pragma unroll
-  for (int st = 0; st < 4; ++st) {
-    const int off = (16 * st + col) * kVaPt + 4 * kg;
-    *reinterpret_cast<uint2*>(pt + off) =
-        make_uint2(pack_bf2(p[st][0], p[st][1]), pack_bf2(p[st][2], p[st][3]));
-  }
+  const float m_new = fmaxf(m, half_max(mx));
+  // A row with no key of its image so far keeps m = -inf: offset 0 then.
+  const float mc = (MASK && m_new == -INFINITY) ? 0.f : m_new * c;
   // Rescale O only when some row's maximum moved (corr == 1 otherwise).
-  if (__builtin_amdgcn_ballot_w64(moved)) {
+  if (__builtin_amdgcn_ballot_w64(m_new != m)) {
+    const float corr = __builtin_amdgcn_exp2f(fmaf(m, c, -mc));
+    lp *= corr;
 #pragma unroll
-    for (int d = 0; d < OT; ++d)
+    for (int d = 0; d < DT; ++d)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[d][i] *= corr[i];
+      for (int r = 0; r < 16; ++r) o[d][r] *= corr;
   }
-  // O += P V over the two 32-key halves; the wave's own LDS stores above
-  // complete before its reads (LDS operations of a wave execute in order).
+  m = m_new;
+  q35_u32x4 p[2];
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    const uint16_t* pth = pt + 32 * half * kVaPt;
-    const uint2 a0 = va_read_tr16(pth + (8 * kg + te) * kVaPt + 4 * tq);
-    const uint2 a1 = va_read_tr16(pth + (8 * kg + 4 + te) * kVaPt + 4 * tq);
-    const uint4 pa = make_uint4(a0.x, a0.y, a1.x, a1.y);
-    // dims 16 d + 4 tq .. +3 of rows r0 and r0 + 4: chunk 2 d + tq / 2, half tq % 2
-    const int r0 = 8 * kg + te;
-    const int g0 = va_swz(r0 & 15), g1 = va_swz((r0 + 4) & 15);
-    const uint16_t* v0 = Vs + (32 * half + r0) * RS + 4 * (tq & 1);
-    const uint16_t* v1 = Vs + (32 * half + r0 + 4) * RS + 4 * (tq & 1);
+  for (int r = 0; r < 16; r += 2) {
+    const float a = __builtin_amdgcn_exp2f(fmaf(s[r], c, -mc)), b = __builtin_amdgcn_exp2f(fmaf(s[r + 1], c, -mc));
+    lp += a + b;
+    p[r >> 3][(r & 7) >> 1] = pack_bf2(a, b);
+  }
+  // dims 32 d + 16 ((lane / 16) % 2) + 4 (lane % 4) of rows 4 kh + e, 4 kh + 8 + e
+  const int e = (lane & 15) >> 2, cl = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+  const int r0 = 4 * kh + e;
+  const int g0 = va_swz(r0), g1 = va_swz(r0 + 8);
 #pragma unroll
-    for (int d = 0; d < OT; ++d) {
-      const int cv = 2 * d + (tq >> 1);
+  for (int kk = 0; kk < 2; ++kk) {
+    const uint16_t* v0 = Vs + (16 * kk + r0) * kVaRS + 4 * (lane & 1);
+    const uint16_t* v1 = v0 + 8 * kVaRS;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      const int cv = 4 * d + cl;
       const uint2 b0 = va_read_tr16(v0 + 8 * (cv ^ g0)), b1 = va_read_tr16(v1 + 8 * (cv ^ g1));
-      o[d] = va_mfma(pa, make_uint4(b0.x, b0.y, b1.x, b1.y), o[d]);
+      o[d] = mfma32(q35_u32x4{b0.x, b0.y, b1.x, b1.y}, p[kk], o[d]);
     }
   }
 }
 
-template <int QT, int OT, int KS>
-__global__ __launch_bounds__(256 * KS) void vision_attn_fa(
+template <int KT, int DT, int KS>
+__global__ __launch_bounds__(256 * KS, 2) void vision_attn_fa(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     uint16_t* __restrict__ out, const int* __restrict__ cu, int nseg, int T, int H, int D,
     float scale) {
-  static_assert(QT >= 1 && QT <= 4 && (OT == 2 * QT || OT == 2 * QT - 1), "head dim tiles");
+  static_assert(DT >= 1 && DT <= 4 && (KT == 2 * DT || KT == 2 * DT - 1), "head dim tiles");
   static_assert(KS == 1 || KS == 2, "key splits");
   constexpr int NT = 256 * KS;         // threads
-  constexpr int SK = kVaKeys * KS;     // keys per stage (one 64-key block per wave group)
-  constexpr int DP = 32 * QT;          // padded head dim
+  constexpr int SK = 64 * KS;          // keys per stage (one 32-key block per wave pair)
+  constexpr int DP = 16 * KT;          // padded head dim
   constexpr int RS = kVaRS;            // LDS row stride (elements), swizzled chunks
   constexpr int NLD = (SK * DP / 8 + NT - 1) / NT;  // 16-byte K (and V) chunks per thread
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int rg = wid & 3;              // 16-row group of the tile
-  const int kh = wid >> 2;             // which block of a stage this wave computes
+  const int rg = wid & 1;              // 32-row group of the tile
+  const int kq = wid >> 1;             // which block of a stage this wave computes
   // Workgroup -> (query tile, head): with heads a multiple of 8 the tiles of a
   // head share one residue mod 8 (one XCD, whose L2 then serves the head's
   // K/V to all of them); otherwise tiles fastest.
@@ -516,9 +493,8 @@ __global__ __launch_bounds__(256 * KS) void vision_attn_fa(
     tile = (int)blockIdx.x % ntiles;
   }
   const int qwg = tile * kVaRows;
-  const int qw0 = qwg + 16 * rg;
-  const int col = lane & 15, kg = lane >> 4;
-  const int te = (lane & 15) >> 2, tq = lane & 3;
+  const int qw0 = qwg + 32 * rg;
+  const int l32 = lane & 31, kh = lane >> 5;
   const int ch = D / 8;            // 16-byte chunks per row
   const float c = scale * 1.4426950408889634f;
   const size_t hb = (size_t)h * T * D;
@@ -529,26 +505,24 @@ __global__ __launch_bounds__(256 * KS) void vision_attn_fa(
   va_segment(cu, nseg, T, qwg, kbeg, tmp);
   va_segment(cu, nseg, T, min(qwg + kVaRows, T) - 1, tmp, kend);
   const int nst = (kend - kbeg + SK - 1) / SK;
-  int s0[4], s1[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) va_segment(cu, nseg, T, min(qw0 + 4 * kg + i, T - 1), s0[i], s1[i]);
+  int s0, s1;
+  va_segment(cu, nseg, T, min(qw0 + l32, T - 1), s0, s1);
   // Keys every row of the wave may see: [latest image start, earliest end).
   int w0, w1;
-  va_segment(cu, nseg, T, min(qw0 + 15, T - 1), w0, tmp);
+  va_segment(cu, nseg, T, min(qw0 + 31, T - 1), w0, tmp);
   va_segment(cu, nseg, T, min(qw0, T - 1), tmp, w1);
 
-  uint4 qa[QT];
+  q35_u32x4 qa[KT];
   {
-    const uint16_t* qrow = q + hb + (size_t)min(qw0 + col, T - 1) * D;
+    const uint16_t* qrow = q + hb + (size_t)min(qw0 + l32, T - 1) * D;
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      const int d0 = 32 * t + 8 * kg;
-      qa[t] = d0 < D ? *reinterpret_cast<const uint4*>(qrow + d0) : make_uint4(0, 0, 0, 0);
+    for (int t = 0; t < KT; ++t) {
+      const int d0 = 16 * t + 8 * kh;
+      qa[t] = d0 < D ? *reinterpret_cast<const q35_u32x4*>(qrow + d0) : q35_u32x4{0u, 0u, 0u, 0u};
     }
   }
 
   __shared__ alignas(16) uint16_t kv_s[2][2][SK * RS];         // [buf][K, V][key][dim]
-  __shared__ alignas(16) uint16_t pt_s[4 * KS][kVaKeys * kVaPt];  // [wave][key][row]
   // Zero the padded dims [D, 128) of every K and V row once (whole 16-byte
   // chunks, at their swizzled places): they meet the zero-padded Q dims in S
   // (0 * finite) and only unused output dims in O.
@@ -596,29 +570,25 @@ __global__ __launch_bounds__(256 * KS) void vision_attn_fa(
       }
     }
   };
-  // This wave's block of stage ST (keys kb..kb+63 of LDS buffer BUF); the
+  // This wave's block of stage ST (keys kb..kb+31 of LDS buffer BUF); the
   // mask is skipped when the block lies inside every row's image.
-#define VA_BLOCK(BUF, ST)                                                                 \
-  do {                                                                                    \
-    const int kb = kbeg + (ST) * SK + kVaKeys * kh;                                       \
-    const uint16_t* Ks = kv_s[BUF][0] + kVaKeys * kh * RS;                                \
-    const uint16_t* Vs = kv_s[BUF][1] + kVaKeys * kh * RS;                                \
-    if (kb >= w0 && kb + kVaKeys <= w1)                                                   \
-      va_block<QT, OT, false>(Ks, Vs, pt, qa, o, m, lp, kb, s0, s1, c, col, kg, te, tq);  \
-    else                                                                                  \
-      va_block<QT, OT, true>(Ks, Vs, pt, qa, o, m, lp, kb, s0, s1, c, col, kg, te, tq);   \
+#define VA_BLOCK(BUF, ST)                                                     \
+  do {                                                                        \
+    const int kb = kbeg + (ST) * SK + 32 * kq;                                \
+    const uint16_t* Ks = kv_s[BUF][0] + 32 * kq * RS;                         \
+    const uint16_t* Vs = kv_s[BUF][1] + 32 * kq * RS;                         \
+    if (kb >= w0 && kb + 32 <= w1)                                            \
+      va_block<KT, DT, false>(Ks, Vs, qa, o, m, lp, kb, s0, s1, c, lane);     \
+    else                                                                      \
+      va_block<KT, DT, true>(Ks, Vs, qa, o, m, lp, kb, s0, s1, c, lane);      \
   } while (0)
 
-  q35_f32x4 o[OT];
+  q35_f32x16 o[DT];
 #pragma unroll
-  for (int d = 0; d < OT; ++d) o[d] = {0.f, 0.f, 0.f, 0.f};
-  float m[4], lp[4];
+  for (int d = 0; d < DT; ++d)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    m[i] = -INFINITY;
-    lp[i] = 0.f;
-  }
-  uint16_t* pt = pt_s[wid];
+    for (int r = 0; r < 16; ++r) o[d][r] = 0.f;
+  float m = -INFINITY, lp = 0.f;
 
   // Two register sets and two LDS buffers: at the top of an iteration LDS
   // buffer 0 holds stage st and set 1 stage st + 1; stage st + 2 is
@@ -644,54 +614,66 @@ __global__ __launch_bounds__(256 * KS) void vision_attn_fa(
   if (st < nst) VA_BLOCK(0, st);
 #undef VA_BLOCK
 
-  if (KS == 2) {
-    // The second wave group hands its (m, partial l, O) to the first through
-    // LDS ([field][row group][lane] floats, conflict-free), which merges
-    // them: both groups hold the same rows and dims lane for lane.
-    constexpr int NF = 4 * OT + 8;
-    static_assert(NF * 4 * 64 * 4 <= (int)sizeof(kv_s), "merge area");
-    float* mg = reinterpret_cast<float*>(&kv_s[0][0][0]);
-    lds_barrier();  // every wave is done with the K/V buffers
-    if (kh == 1) {
+  // The other key groups hand their (m, partial l, O) to the first through
+  // LDS ([group][row group][field][lane], conflict-free), which merges them:
+  // all groups hold the same rows and dims lane for lane.
+  constexpr int NF = 4 * DT + 1;  // 16-byte fields
+  static_assert((2 * KS - 1) * 2 * NF * 64 * 16 <= (int)sizeof(kv_s), "merge area");
+  float4* mg = reinterpret_cast<float4*>(&kv_s[0][0][0]);
+  lds_barrier();  // every wave is done with the K/V buffers
+  if (kq) {
+    float4* f = mg + ((kq - 1) * 2 + rg) * NF * 64 + lane;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        mg[((i) * 4 + rg) * 64 + lane] = m[i];
-        mg[((4 + i) * 4 + rg) * 64 + lane] = lp[i];
+    for (int d = 0; d < DT; ++d)
 #pragma unroll
-        for (int d = 0; d < OT; ++d) mg[((8 + 4 * d + i) * 4 + rg) * 64 + lane] = o[d][i];
+      for (int u = 0; u < 4; ++u)
+        f[(4 * d + u) * 64] = make_float4(o[d][4 * u], o[d][4 * u + 1], o[d][4 * u + 2], o[d][4 * u + 3]);
+    f[4 * DT * 64] = make_float4(m, lp, 0.f, 0.f);
+  }
+  lds_barrier();
+  if (kq) return;
+  for (int g = 0; g < 2 * KS - 1; ++g) {
+    const float4* f = mg + (g * 2 + rg) * NF * 64 + lane;
+    const float4 ml = f[4 * DT * 64];
+    const float mm = fmaxf(m, ml.x);
+    const float msub = mm == -INFINITY ? 0.f : mm * c;
+    const float f0 = __builtin_amdgcn_exp2f(fmaf(m, c, -msub));
+    const float f1 = __builtin_amdgcn_exp2f(fmaf(ml.x, c, -msub));
+    m = mm;
+    lp = lp * f0 + ml.y * f1;
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float4 x = f[(4 * d + u) * 64];
+        o[d][4 * u] = o[d][4 * u] * f0 + x.x * f1;
+        o[d][4 * u + 1] = o[d][4 * u + 1] * f0 + x.y * f1;
+        o[d][4 * u + 2] = o[d][4 * u + 2] * f0 + x.z * f1;
+        o[d][4 * u + 3] = o[d][4 * u + 3] * f0 + x.w * f1;
+      }
+  }
+  const float inv = 1.0f / half_sum(lp);
+  const int row = qw0 + l32;
+  if (row >= T) return;
+  uint16_t* orow = out + (size_t)row * H * D + (size_t)h * D;
+  const bool vec = ((uintptr_t)out & 7) == 0;
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int dim = 32 * d + 8 * u + 4 * kh;
+      if (dim >= D) continue;
+      const uint2 v2 = make_uint2(pack_bf2(o[d][4 * u] * inv, o[d][4 * u + 1] * inv),
+                                  pack_bf2(o[d][4 * u + 2] * inv, o[d][4 * u + 3] * inv));
+      if (vec) {
+        *reinterpret_cast<uint2*>(orow + dim) = v2;
+      } else {
+        orow[dim] = (uint16_t)v2.x;
+        orow[dim + 1] = (uint16_t)(v2.x >> 16);
+        orow[dim + 2] = (uint16_t)v2.y;
+        orow[dim + 3] = (uint16_t)(v2.y >> 16);
       }
     }
-    lds_barrier();
-    if (kh == 1) return;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float m1 = mg[((i) * 4 + rg) * 64 + lane];
-      const float l1 = mg[((4 + i) * 4 + rg) * 64 + lane];
-      const float mm = fmaxf(m[i], m1);
-      const float msub = mm == -INFINITY ? 0.f : mm * c;
-      const float f0 = __builtin_amdgcn_exp2f(fmaf(m[i], c, -msub));
-      const float f1 = __builtin_amdgcn_exp2f(fmaf(m1, c, -msub));
-      lp[i] = lp[i] * f0 + l1 * f1;
-#pragma unroll
-      for (int d = 0; d < OT; ++d)
-        o[d][i] = o[d][i] * f0 + mg[((8 + 4 * d + i) * 4 + rg) * 64 + lane] * f1;
-    }
-  }
-  const size_t ostride = (size_t)H * D;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float l = row16_sum(lp[i]);
-    const int r = qw0 + 4 * kg + i;
-    if (r < T) {
-      const float inv = 1.0f / l;
-      uint16_t* orow = out + (size_t)r * ostride + (size_t)h * D;
-#pragma unroll
-      for (int d = 0; d < OT; ++d) {
-        const int dim = 16 * d + col;
-        if (dim < D) orow[dim] = (uint16_t)f2bf(o[d][i] * inv);
-      }
-    }
-  }
 }
 
 }  // namespace
@@ -767,29 +749,28 @@ int q35_vision_attention(const void* q, const void* k, const void* v, void* out,
   const int* cu = (const int*)cu_seqlens;
   const uint16_t *qs = (const uint16_t*)q, *ks = (const uint16_t*)k, *vs = (const uint16_t*)v;
   uint16_t* os = (uint16_t*)out;
-  const int qt = (dim + 31) / 32, ot = (dim + 15) / 16;
-#define VA_LAUNCH(QT_, OT_, KS_)                                                          \
-  vision_attn_fa<QT_, OT_, KS_><<<grid, 256 * KS_, 0, stream>>>(qs, ks, vs, os, cu, n_images, \
-                                                                tokens, heads, dim, scale)
-  // Two key blocks per stage (8 waves, one workgroup per CU by LDS) while the
-  // grid leaves CUs idle; one block (4 waves, two workgroups per CU) for
-  // larger grids and for the 128-dim tiles, whose registers do not fit two
-  // waves per SIMD.
+  const int kt = (dim + 15) / 16;
+#define VA_LAUNCH(KT_, KS_)                                                                  \
+  vision_attn_fa<KT_, (KT_ + 1) / 2, KS_><<<grid, 256 * KS_, 0, stream>>>(qs, ks, vs, os, cu, \
+                                                                          n_images, tokens, heads, dim, scale)
+  // 128 keys per stage (8 waves, one workgroup per CU by LDS) while the grid
+  // leaves CUs idle; 64 (4 waves, two workgroups per CU) for larger grids and
+  // for the 128-dim tiles, whose registers do not fit two waves per SIMD.
   const bool split = grid < 512;
-#define VA_PICK(QT_, OT_)        \
-  if (split)                     \
-    VA_LAUNCH(QT_, OT_, 2);      \
-  else                           \
-    VA_LAUNCH(QT_, OT_, 1);
-  switch (qt * 8 + ot) {
-    case 1 * 8 + 1: VA_PICK(1, 1); break;
-    case 1 * 8 + 2: VA_PICK(1, 2); break;
-    case 2 * 8 + 3: VA_PICK(2, 3); break;
-    case 2 * 8 + 4: VA_PICK(2, 4); break;
-    case 3 * 8 + 5: VA_PICK(3, 5); break;
-    case 3 * 8 + 6: VA_PICK(3, 6); break;
-    case 4 * 8 + 7: VA_LAUNCH(4, 7, 1); break;
-    default: VA_LAUNCH(4, 8, 1); break;
+#define VA_PICK(KT_)      \
+  if (split)              \
+    VA_LAUNCH(KT_, 2);    \
+  else                    \
+    VA_LAUNCH(KT_, 1);
+  switch (kt) {
+    case 1: VA_PICK(1); break;
+    case 2: VA_PICK(2); break;
+    case 3: VA_PICK(3); break;
+    case 4: VA_PICK(4); break;
+    case 5: VA_PICK(5); break;
+    case 6: VA_PICK(6); break;
+    case 7: VA_LAUNCH(7, 1); break;
+    default: VA_LAUNCH(8, 1); break;
   }
 #undef VA_PICK
 #undef VA_LAUNCH
