@@ -658,6 +658,554 @@ void launch_combine(const float* acc, const float* ml, const uint16_t* gate, uin
     gqa_decode_combine<8><<<grid, 256, 0, stream>>>(acc, ml, gate, out, splits, advance);
 }
 
+// ------------------------------------------------- causal prefill (MFMA)
+// Flash attention on the matrix cores, v_mfma_f32_16x16x32_bf16. Operand
+// layouts (wave64): A[16 x 32]: lane l holds row l%16, 8 consecutive k at
+// 8*(l/16); B[32 x 16]: lane l holds column l%16, the same 8 k; C[16 x 16]:
+// lane l holds rows 4*(l/16) + i (i = 0..3) of column l%16.
+// Grid (query tiles of 16 rows, KVH, B); the G waves of a workgroup are the G
+// query heads of one KV head over the same 16 rows, so they share the K rows
+// (L1) and the V tile (LDS). Per 32-key iteration and wave:
+//   S = Q K^T: Q (A operand, rows x dims) stays in registers, K rows are the
+//     B operand in their natural layout (16 contiguous bytes per lane);
+//   online softmax on the C layout (row max / sum over the 16 lanes of a DPP
+//     row), scale and causal mask applied to S in fp32;
+//   O += P V: P is split into bf16 hi + lo parts (p - hi rounded again, so P
+//     keeps ~16 mantissa bits: two MFMAs instead of the one of a plain bf16 P)
+//     and moved through a wave-private LDS tile into the A layout; V is staged
+//     transposed in LDS (double-buffered, one barrier per iteration) so the
+//     B operand is again 16 contiguous bytes per lane.
+// Keys past the valid end are masked to -inf and their V rows staged as
+// zeros (the cache beyond the prompt may hold any bits).
+Q35_DEV q35_f32x4 mfma_16x16x32(const uint4 a, const uint4 b, q35_f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(q35_bf16x8, a),
+                                                 __builtin_bit_cast(q35_bf16x8, b), c, 0, 0, 0);
+}
+
+constexpr int kVtStride = 40;  // bf16 per transposed V row: 32 keys + pad
+constexpr int kPStride = 40;   // bf16 per P row: 32 keys + pad
+
+template <int G>
+__global__ __launch_bounds__(G * 64) void gqa_prefill_mfma(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc, const uint16_t* __restrict__ Vc,
+    uint16_t* __restrict__ out, int B, int QH, int KVH, int L, int cache_len, int kv_start_host,
+    const long long* __restrict__ valid_len, float scale) {
+  const int lane = threadIdx.x & 63;
+  const int wid = threadIdx.x >> 6;
+  const int tile = gridDim.x - 1 - blockIdx.x;  // heavy (late) tiles first
+  const int kvh = blockIdx.y;
+  const int b = blockIdx.z;
+  const int h = kvh * G + wid;
+  const int q0 = tile * 16;
+  long long ks = valid_len ? valid_len[0] - L + kv_start_host : (long long)kv_start_host;
+  if (ks < 0) ks = 0;
+  if (ks + L > cache_len) ks = cache_len - L;
+  const int kv_start = (int)ks;
+  const int col = lane & 15;  // A row / B column / C column
+  const int kg = lane >> 4;   // k group of 8 / C row group of 4
+
+  // Q operand: row q0 + col (clamped), dims 8*kg + 32t.
+  const uint16_t* qp = q + (((size_t)b * QH + h) * L + min(q0 + col, L - 1)) * kAD + kg * 8;
+  uint4 qa[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) qa[t] = *reinterpret_cast<const uint4*>(qp + 32 * t);
+  int row_abs[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) row_abs[i] = kv_start + min(q0 + 4 * kg + i, L - 1);
+  const int n_keys = min(kv_start + min(q0 + 16, L), cache_len);
+  const uint16_t* Kh = Kc + ((size_t)b * KVH + kvh) * cache_len * kAD;
+  const uint16_t* Vh = Vc + ((size_t)b * KVH + kvh) * cache_len * kAD;
+
+  __shared__ alignas(16) uint16_t vt_s[2][kAD * kVtStride];
+  __shared__ alignas(16) uint16_t p_s[G][2][16 * kPStride];
+  q35_f32x4 o[16];
+#pragma unroll
+  for (int d = 0; d < 16; ++d) o[d] = {0.f, 0.f, 0.f, 0.f};
+  float m[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m[i] = -INFINITY;
+    l[i] = 0.f;
+  }
+  const int nblk = (n_keys + 31) / 32;
+  // Global loads of one 32-key block: the K operand of its two 16-key halves
+  // (key kb + 16*sb + col, dims 8*kg + 32t) and this thread's share of V rows
+  // for the transposed staging. Block blk + 1 is requested before block blk
+  // is computed, so the loop does not wait on memory.
+  constexpr int VPER = (32 * (kAD / 8) + G * 64 - 1) / (G * 64);
+  auto load_block = [&](int blk, uint4 (&kv)[2][8], uint4 (&vr)[VPER]) {
+    const int kb = blk * 32;
+#pragma unroll
+    for (int sb = 0; sb < 2; ++sb) {
+      const uint16_t* kr = Kh + (size_t)min(kb + 16 * sb + col, n_keys - 1) * kAD + kg * 8;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) kv[sb][t] = *reinterpret_cast<const uint4*>(kr + 32 * t);
+    }
+#pragma unroll
+    for (int j = 0; j < VPER; ++j) {
+      const int pi = min((int)threadIdx.x + j * G * 64, 32 * (kAD / 8) - 1);
+      const int k = pi & 31, dg = pi >> 5;
+      vr[j] = *reinterpret_cast<const uint4*>(Vh + (size_t)min(kb + k, n_keys - 1) * kAD + dg * 8);
+    }
+  };
+  uint4 kv[2][8], vr[VPER];
+  load_block(0, kv, vr);
+  for (int blk = 0; blk < nblk; ++blk) {
+    const int kb = blk * 32;
+    uint16_t* vt = vt_s[blk & 1];
+    uint4 kn[2][8], vn[VPER];
+    load_block(min(blk + 1, nblk - 1), kn, vn);
+    // Stage V^T: (key, 8-dim group) pairs, vt[dim][key]; masked keys as zeros.
+#pragma unroll
+    for (int j = 0; j < VPER; ++j) {
+      const int pi = (int)threadIdx.x + j * G * 64;
+      if (pi < 32 * (kAD / 8)) {
+        const int k = pi & 31, dg = pi >> 5;
+        const uint4 v = kb + k < n_keys ? vr[j] : make_uint4(0, 0, 0, 0);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          vt[(dg * 8 + 2 * e) * kVtStride + k] = (uint16_t)(w[e] & 0xffffu);
+          vt[(dg * 8 + 2 * e + 1) * kVtStride + k] = (uint16_t)(w[e] >> 16);
+        }
+      }
+    }
+    // S = Q K^T, then scale, causal mask and online softmax per row.
+    q35_f32x4 s[2];
+#pragma unroll
+    for (int sb = 0; sb < 2; ++sb) {
+      s[sb] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 8; ++t) s[sb] = mfma_16x16x32(qa[t], kv[sb][t], s[sb]);
+    }
+    float corr[4];
+    uint16_t* ps_hi = p_s[wid][0];
+    uint16_t* ps_lo = p_s[wid][1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float sv[2];
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb) {
+        const int key = kb + 16 * sb + col;
+        sv[sb] = (key <= row_abs[i] && key < n_keys) ? s[sb][i] * scale : -INFINITY;
+      }
+      const float m_new = fmaxf(m[i], row16_max(fmaxf(sv[0], sv[1])));
+      // A row without any valid key so far keeps m = -inf: subtract 0 then.
+      const float m_sub = m_new == -INFINITY ? 0.f : m_new;
+      corr[i] = expf(m[i] - m_sub);
+      const float p0 = expf(sv[0] - m_sub), p1 = expf(sv[1] - m_sub);
+      l[i] = l[i] * corr[i] + row16_sum(p0 + p1);
+      m[i] = m_new;
+      const uint32_t h0 = f2bf(p0), h1 = f2bf(p1);
+      ps_hi[(4 * kg + i) * kPStride + col] = (uint16_t)h0;
+      ps_hi[(4 * kg + i) * kPStride + 16 + col] = (uint16_t)h1;
+      ps_lo[(4 * kg + i) * kPStride + col] = (uint16_t)f2bf(p0 - bf2f(h0));
+      ps_lo[(4 * kg + i) * kPStride + 16 + col] = (uint16_t)f2bf(p1 - bf2f(h1));
+    }
+    __syncthreads();  // V^T staged by every wave; this wave's P tile written
+    // O += P V: A = P rows x keys (row col, keys 8*kg..), B = V^T (dims x keys).
+    const uint4 pa_hi = *reinterpret_cast<const uint4*>(ps_hi + col * kPStride + kg * 8);
+    const uint4 pa_lo = *reinterpret_cast<const uint4*>(ps_lo + col * kPStride + kg * 8);
+#pragma unroll
+    for (int d = 0; d < 16; ++d) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[d][i] *= corr[i];
+      const uint4 vb = *reinterpret_cast<const uint4*>(vt + (d * 16 + col) * kVtStride + kg * 8);
+      o[d] = mfma_16x16x32(pa_hi, vb, o[d]);
+      o[d] = mfma_16x16x32(pa_lo, vb, o[d]);
+    }
+#pragma unroll
+    for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+      for (int t = 0; t < 8; ++t) kv[sb][t] = kn[sb][t];
+#pragma unroll
+    for (int j = 0; j < VPER; ++j) vr[j] = vn[j];
+  }
+  // out[b, row, h*D + 16d + col] = bf16(O / l) for the valid rows.
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = q0 + 4 * kg + i;
+    if (r < L) {
+      const float inv = 1.0f / l[i];
+      uint16_t* orow = out + ((size_t)b * L + r) * QH * kAD + h * kAD + col;
+#pragma unroll
+      for (int d = 0; d < 16; ++d) orow[16 * d] = (uint16_t)f2bf(o[d][i] * inv);
+    }
+  }
+}
+
+// ------------------------------------------ causal prefill, 64-key blocks
+// Grid (query tiles of 16 rows, heavy first; KVH; B). A workgroup has 2G
+// waves: wave w serves query head g = w % G of the KV head over key half
+// kh = w / G (keys 32kh..32kh+31 of every 64-key block), with its own online
+// softmax; the two halves of a head are merged in LDS at the end. Per block
+// the K and V rows are staged once for all waves in their natural [key][dim]
+// layout (16-byte stores, double-buffered, one barrier per block; the next
+// block is loaded to registers before the current one is computed).
+//   S = Q K^T: Q rows (A operand) stay in registers, K rows are read from LDS
+//     as the B operand (16 contiguous bytes per lane);
+//   O += P V: P is kept as bf16 hi + lo (~16 mantissa bits, two MFMAs); the
+//     wave writes P^T [key][row] (4 rows = 8 bytes per lane) and reads the A
+//     operand back with the gfx950 transpose read ds_read_b64_tr_b16, which
+//     also turns row-major V into the B operand. Within each 16-lane group g
+//     the read returns to lane 16g + i, element e, the 16-bit word at
+//     address(lane 16g + 4e + i/4) + (i % 4); so lane 16g + 4e + q pointing at
+//     row 8g + 4h + e, column 16t + 4q gives lane 16g + i the 4 rows
+//     8g + 4h .. 8g + 4h + 3 of column 16t + i: read h = 0, 1 fill the 8
+//     consecutive k of an MFMA operand.
+// Keys past the valid end are clamped to the last valid row on load (finite
+// values) and masked to -inf in S, so they add exact zeros.
+typedef short q35_i16x4 __attribute__((ext_vector_type(4)));
+Q35_DEV uint2 lds_read_tr16(const uint16_t* p) {
+  const q35_i16x4 v =
+      __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) q35_i16x4*)(p));
+  return __builtin_bit_cast(uint2, v);
+}
+
+constexpr int kFaKeys = 64;         // keys per block
+constexpr int kFaRow = kAD + 16;    // padded K/V row in LDS (elements)
+constexpr int kFaPt = 16 + 4;       // padded P^T row (16 query rows)
+
+template <int G>
+__global__ __launch_bounds__(2 * G * 64) void gqa_prefill_fa(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc, const uint16_t* __restrict__ Vc,
+    uint16_t* __restrict__ out, int B, int QH, int KVH, int L, int cache_len, int kv_start_host,
+    const long long* __restrict__ valid_len, float scale, int sb, int smax,
+    float* __restrict__ part) {
+  constexpr int NW = 2 * G;
+  constexpr int NT = NW * 64;
+  constexpr int PER = kFaKeys * (kAD / 8) / NT;  // 16-byte K (and V) groups per thread
+  static_assert(PER * NT == kFaKeys * (kAD / 8), "block must split evenly");
+  const int lane = threadIdx.x & 63;
+  const int wid = threadIdx.x >> 6;
+  const int g = wid % G, kh = wid / G;
+  const int ntiles = gridDim.x / smax;
+  const int tile = ntiles - 1 - (int)blockIdx.x / smax;  // heavy (late) tiles first
+  const int split = (int)blockIdx.x % smax;
+  const int kvh = blockIdx.y;
+  const int b = blockIdx.z;
+  const int h = kvh * G + g;
+  const int q0 = tile * 16;
+  long long ks = valid_len ? valid_len[0] - L + kv_start_host : (long long)kv_start_host;
+  if (ks < 0) ks = 0;
+  if (ks + L > cache_len) ks = cache_len - L;
+  const int kv_start = (int)ks;
+  const int col = lane & 15;  // A row / B column / C column
+  const int kg = lane >> 4;   // k group of 8 / C row group of 4
+  // transpose-read addressing: lane 16*kg + 4e + tq reads row 4e-offset, column 4tq
+  const int te = (lane & 15) >> 2, tq = lane & 3;
+
+  const uint16_t* qp = q + (((size_t)b * QH + h) * L + min(q0 + col, L - 1)) * kAD + kg * 8;
+  uint4 qa[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) qa[t] = *reinterpret_cast<const uint4*>(qp + 32 * t);
+  int row_abs[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) row_abs[i] = kv_start + min(q0 + 4 * kg + i, L - 1);
+  const int n_keys = min(kv_start + min(q0 + 16, L), cache_len);
+  const int nblk = (n_keys + kFaKeys - 1) / kFaKeys;
+  // This workgroup's key blocks [b0, b1) of the tile (sb blocks per split).
+  const int nsplit = (nblk + sb - 1) / sb;
+  if (split >= nsplit) return;  // whole workgroup: no barrier is skipped
+  const int b0 = split * sb, b1 = min(b0 + sb, nblk);
+  const uint16_t* Kh = Kc + ((size_t)b * KVH + kvh) * cache_len * kAD;
+  const uint16_t* Vh = Vc + ((size_t)b * KVH + kvh) * cache_len * kAD;
+
+  __shared__ alignas(16) uint16_t kv_s[2][2][kFaKeys * kFaRow];  // [buf][K, V][key][dim]
+  __shared__ alignas(16) uint16_t pt_s[NW][2][32 * kFaPt];       // [wave][hi, lo][key][row]
+
+  uint4 kr[PER], vr[PER];
+#define Q35_FA_LOAD(blk)                                                                 \
+  do {                                                                                   \
+    _Pragma("unroll") for (int j = 0; j < PER; ++j) {                                     \
+      const int gi = (int)threadIdx.x + j * NT;                                           \
+      const int key = min((blk) * kFaKeys + (gi >> 5), n_keys - 1);                       \
+      const size_t off = (size_t)key * kAD + (gi & 31) * 8;                               \
+      kr[j] = *reinterpret_cast<const uint4*>(Kh + off);                                  \
+      vr[j] = *reinterpret_cast<const uint4*>(Vh + off);                                  \
+    }                                                                                     \
+  } while (0)
+#define Q35_FA_STORE(buf)                                                                \
+  do {                                                                                   \
+    _Pragma("unroll") for (int j = 0; j < PER; ++j) {                                     \
+      const int gi = (int)threadIdx.x + j * NT;                                           \
+      const int off = (gi >> 5) * kFaRow + (gi & 31) * 8;                                 \
+      *reinterpret_cast<uint4*>(&kv_s[buf][0][off]) = kr[j];                              \
+      *reinterpret_cast<uint4*>(&kv_s[buf][1][off]) = vr[j];                              \
+    }                                                                                     \
+  } while (0)
+
+  q35_f32x4 o[16];
+#pragma unroll
+  for (int d = 0; d < 16; ++d) o[d] = {0.f, 0.f, 0.f, 0.f};
+  float m[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m[i] = -INFINITY;
+    l[i] = 0.f;
+  }
+  uint16_t* pt_hi = pt_s[wid][0];
+  uint16_t* pt_lo = pt_s[wid][1];
+
+  Q35_FA_LOAD(b0);
+  Q35_FA_STORE(0);
+  __syncthreads();
+  for (int blk = b0; blk < b1; ++blk) {
+    const int buf = (blk - b0) & 1;
+    Q35_FA_LOAD(min(blk + 1, b1 - 1));  // in flight while this block is computed
+    const uint16_t* Ks = kv_s[buf][0] + 32 * kh * kFaRow;
+    const uint16_t* Vs = kv_s[buf][1] + 32 * kh * kFaRow;
+    const int kb = blk * kFaKeys + 32 * kh;  // first key of this wave's half
+    // S = Q K^T over the wave's 32 keys (two 16-key column tiles).
+    q35_f32x4 s[2];
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      s[st] = {0.f, 0.f, 0.f, 0.f};
+      const uint16_t* krow = Ks + (16 * st + col) * kFaRow + 8 * kg;
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        s[st] = mfma_16x16x32(qa[t], *reinterpret_cast<const uint4*>(krow + 32 * t), s[st]);
+    }
+    // Online softmax per row; P^T as bf16 hi + lo, 4 rows (8 bytes) per store.
+    float corr[4], p[2][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float sv[2];
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const int key = kb + 16 * st + col;
+        sv[st] = (key <= row_abs[i] && key < n_keys) ? s[st][i] * scale : -INFINITY;
+      }
+      const float m_new = fmaxf(m[i], row16_max(fmaxf(sv[0], sv[1])));
+      // A row without any valid key so far keeps m = -inf: subtract 0 then.
+      const float m_sub = m_new == -INFINITY ? 0.f : m_new;
+      corr[i] = expf(m[i] - m_sub);
+      p[0][i] = expf(sv[0] - m_sub);
+      p[1][i] = expf(sv[1] - m_sub);
+      l[i] = l[i] * corr[i] + row16_sum(p[0][i] + p[1][i]);
+      m[i] = m_new;
+    }
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      float hi[4], lo[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        hi[i] = round_bf(p[st][i]);
+        lo[i] = p[st][i] - hi[i];
+      }
+      const int off = (16 * st + col) * kFaPt + 4 * kg;
+      *reinterpret_cast<uint2*>(pt_hi + off) = make_uint2(pack_bf2(hi[0], hi[1]), pack_bf2(hi[2], hi[3]));
+      *reinterpret_cast<uint2*>(pt_lo + off) = make_uint2(pack_bf2(lo[0], lo[1]), pack_bf2(lo[2], lo[3]));
+    }
+    // P operand (rows x 32 keys) back through the transpose read; the wave's
+    // own LDS stores above complete before its later reads (in-order LDS).
+    uint4 pa_hi, pa_lo;
+    {
+      const int off0 = (8 * kg + te) * kFaPt + 4 * tq;
+      const int off1 = (8 * kg + 4 + te) * kFaPt + 4 * tq;
+      const uint2 h0 = lds_read_tr16(pt_hi + off0), h1 = lds_read_tr16(pt_hi + off1);
+      const uint2 l0 = lds_read_tr16(pt_lo + off0), l1 = lds_read_tr16(pt_lo + off1);
+      pa_hi = make_uint4(h0.x, h0.y, h1.x, h1.y);
+      pa_lo = make_uint4(l0.x, l0.y, l1.x, l1.y);
+    }
+    // O += P V; V rows 8kg + 4h + te of the wave's half, dims 16d + 4tq.
+    const uint16_t* v0 = Vs + (8 * kg + te) * kFaRow + 4 * tq;
+    const uint16_t* v1 = Vs + (8 * kg + 4 + te) * kFaRow + 4 * tq;
+#pragma unroll
+    for (int d = 0; d < 16; ++d) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[d][i] *= corr[i];
+      const uint2 a = lds_read_tr16(v0 + 16 * d), c = lds_read_tr16(v1 + 16 * d);
+      const uint4 vb = make_uint4(a.x, a.y, c.x, c.y);
+      o[d] = mfma_16x16x32(pa_hi, vb, o[d]);
+      o[d] = mfma_16x16x32(pa_lo, vb, o[d]);
+    }
+    Q35_FA_STORE(buf ^ 1);
+    __syncthreads();
+  }
+#undef Q35_FA_LOAD
+#undef Q35_FA_STORE
+
+  // Merge the two key halves of each head: half 1 leaves (O, m, l) in LDS
+  // (the K/V buffers are free after the last barrier), half 0 combines and
+  // writes out[b, row, h*D + 16d + col] = bf16(O / l) for the valid rows.
+  float* mo = reinterpret_cast<float*>(&kv_s[0][0][0]);  // [G][16 rows][kAD]
+  float* ml = mo + G * 16 * kAD;                           // [G][16 rows][2]
+  if (kh == 1) {
+#pragma unroll
+    for (int d = 0; d < 16; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mo[(g * 16 + 4 * kg + i) * kAD + 16 * d + col] = o[d][i];
+    if (col == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ml[(g * 16 + 4 * kg + i) * 2] = m[i];
+        ml[(g * 16 + 4 * kg + i) * 2 + 1] = l[i];
+      }
+    }
+  }
+  __syncthreads();
+  if (kh == 0) {
+    // One split: the final rows. Several: this split's (O, m, l) record, O
+    // relative to m and not yet divided by l; gqa_prefill_merge combines them.
+    float* rec = nsplit > 1 ? part + ((((size_t)b * KVH + kvh) * ntiles + tile) * smax + split) *
+                                         (size_t)(G * 16 * (kAD + 2))
+                            : nullptr;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = q0 + 4 * kg + i;
+      const int rr = g * 16 + 4 * kg + i;
+      const float m1 = ml[rr * 2], l1 = ml[rr * 2 + 1];
+      const float mm = fmaxf(m[i], m1);
+      const float f0 = m[i] == -INFINITY ? 0.f : expf(m[i] - mm);
+      const float f1 = m1 == -INFINITY ? 0.f : expf(m1 - mm);
+      const float lt = l[i] * f0 + l1 * f1;
+      if (rec) {
+#pragma unroll
+        for (int d = 0; d < 16; ++d)
+          rec[rr * kAD + 16 * d + col] = o[d][i] * f0 + mo[rr * kAD + 16 * d + col] * f1;
+        if (col == 0) {
+          rec[G * 16 * kAD + rr * 2] = mm;
+          rec[G * 16 * kAD + rr * 2 + 1] = lt;
+        }
+      } else if (r < L) {
+        const float inv = 1.0f / lt;
+        uint16_t* orow = out + ((size_t)b * L + r) * QH * kAD + h * kAD + col;
+#pragma unroll
+        for (int d = 0; d < 16; ++d) {
+          const float v = o[d][i] * f0 + mo[rr * kAD + 16 * d + col] * f1;
+          orow[16 * d] = (uint16_t)f2bf(v * inv);
+        }
+      }
+    }
+  }
+}
+
+// Merge of the split records of the query tiles with more than one split:
+// one thread per (query head g, row r, 16 dims), G*256 threads per (tile, KV
+// head); O = sum_s O_s e^{m_s - M} / sum_s l_s e^{m_s - M}, M = max_s m_s.
+template <int G>
+__global__ __launch_bounds__(G * 256) void gqa_prefill_merge(
+    const float* __restrict__ part, uint16_t* __restrict__ out, int B, int QH, int KVH, int L,
+    int cache_len, int kv_start_host, const long long* __restrict__ valid_len, int sb, int smax) {
+  const int t = threadIdx.x;
+  const int g = t >> 8, r = (t >> 4) & 15, dq = t & 15;
+  const int tile = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  const int ntiles = gridDim.x;
+  const int q0 = tile * 16;
+  long long ks = valid_len ? valid_len[0] - L + kv_start_host : (long long)kv_start_host;
+  if (ks < 0) ks = 0;
+  if (ks + L > cache_len) ks = cache_len - L;
+  const int n_keys = min((int)ks + min(q0 + 16, L), cache_len);
+  const int nblk = (n_keys + kFaKeys - 1) / kFaKeys;
+  const int nsplit = (nblk + sb - 1) / sb;
+  if (nsplit <= 1 || q0 + r >= L) return;  // no barrier in this kernel
+  const size_t rs = (size_t)G * 16 * (kAD + 2);
+  const float* rec0 = part + (((size_t)b * KVH + kvh) * ntiles + tile) * smax * rs;
+  const int rr = g * 16 + r;
+  float mx = -INFINITY;
+  for (int sp = 0; sp < nsplit; ++sp) mx = fmaxf(mx, rec0[sp * rs + G * 16 * kAD + rr * 2]);
+  float acc[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+  float lt = 0.f;
+  for (int sp = 0; sp < nsplit; ++sp) {
+    const float* rec = rec0 + sp * rs;
+    const float ms = rec[G * 16 * kAD + rr * 2];
+    const float f = ms == -INFINITY ? 0.f : expf(ms - mx);
+    lt += rec[G * 16 * kAD + rr * 2 + 1] * f;
+    const float4* v = reinterpret_cast<const float4*>(rec + rr * kAD + 16 * dq);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 x = v[j];
+      acc[4 * j] = fmaf(x.x, f, acc[4 * j]);
+      acc[4 * j + 1] = fmaf(x.y, f, acc[4 * j + 1]);
+      acc[4 * j + 2] = fmaf(x.z, f, acc[4 * j + 2]);
+      acc[4 * j + 3] = fmaf(x.w, f, acc[4 * j + 3]);
+    }
+  }
+  const float inv = 1.0f / lt;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] *= inv;
+  uint4* o = reinterpret_cast<uint4*>(out + ((size_t)b * L + q0 + r) * QH * kAD + (kvh * G + g) * kAD + 16 * dq);
+  o[0] = pack8(acc);
+  o[1] = pack8(acc + 8);
+}
+
+// ---------------------------------------------------------- causal prefill
+// q [B, QH, L, D], K/V [B, KVH, cache_len, D] (the prompt at cache offset
+// kv_start), out [B, L, QH*D]. Query row i of a head attends to keys
+// [0, kv_start + i]. One wave per (batch, head, query row); 4 keys per
+// iteration, lane = (key kk = lane/16, 16-dim slice); online softmax in fp32.
+__global__ __launch_bounds__(256) void gqa_prefill_rows(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ Kc, const uint16_t* __restrict__ Vc,
+    uint16_t* __restrict__ out, int B, int QH, int KVH, int L, int cache_len, int kv_start_host,
+    const long long* __restrict__ valid_len, float scale) {
+  const int lane = threadIdx.x & 63;
+  const long long wv = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (wv >= (long long)B * QH * L) return;
+  // With a device length the prompt starts at valid_len - L + kv_start
+  // (kv_start = 0 when the length already counts these L tokens, L when it
+  // holds the start); the bound keeps reads in the cache.
+  long long ks = valid_len ? valid_len[0] - L + kv_start_host : (long long)kv_start_host;
+  if (ks < 0) ks = 0;
+  if (ks + L > cache_len) ks = cache_len - L;
+  const int kv_start = (int)ks;
+  // Heavy (late) rows first so that the tail of the grid is short.
+  const int i = L - 1 - (int)(wv % L);
+  const int h = (int)((wv / L) % QH);
+  const int b = (int)(wv / ((long long)L * QH));
+  const int kvh = h / (QH / KVH);
+  const int ds = lane & 15;
+  const uint16_t* qr = q + (((size_t)b * QH + h) * L + i) * kAD + ds * 16;
+  float qf[16], t8[8];
+  unpack8(*reinterpret_cast<const uint4*>(qr), t8);
+  for (int j = 0; j < 8; ++j) qf[j] = t8[j] * scale;
+  unpack8(*reinterpret_cast<const uint4*>(qr + 8), t8);
+  for (int j = 0; j < 8; ++j) qf[8 + j] = t8[j] * scale;
+  const uint16_t* Kh = Kc + ((size_t)b * KVH + kvh) * cache_len * kAD;
+  const uint16_t* Vh = Vc + ((size_t)b * KVH + kvh) * cache_len * kAD;
+  const int n = kv_start + i + 1;
+  float m = -INFINITY, l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int t0 = 0; t0 < n; t0 += 4) {
+    const int tok = t0 + (lane >> 4);
+    const bool live = tok < n;
+    float s = 0.f;
+    if (live) {
+      const uint16_t* kr = Kh + (size_t)tok * kAD + ds * 16;
+      unpack8(*reinterpret_cast<const uint4*>(kr), t8);
+      for (int j = 0; j < 8; ++j) s = fmaf(qf[j], t8[j], s);
+      unpack8(*reinterpret_cast<const uint4*>(kr + 8), t8);
+      for (int j = 0; j < 8; ++j) s = fmaf(qf[8 + j], t8[j], s);
+    }
+    uint2 vv[4];
+    for (int k = 0; k < 4; ++k)
+      vv[k] = t0 + k < n ? *reinterpret_cast<const uint2*>(Vh + (size_t)(t0 + k) * kAD + 4 * lane)
+                         : make_uint2(0, 0);
+    s = row16_sum(s);
+    s = live ? s : -INFINITY;
+    float sc[4];
+    for (int k = 0; k < 4; ++k) sc[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), 16 * k));
+    const float m_new = fmaxf(m, fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])));
+    const float corr = expf(m - m_new);
+    float p[4];
+    for (int k = 0; k < 4; ++k) p[k] = expf(sc[k] - m_new);
+    l = l * corr + ((p[0] + p[1]) + (p[2] + p[3]));
+    for (int d = 0; d < 4; ++d) acc[d] *= corr;
+    for (int k = 0; k < 4; ++k) {
+      acc[0] = fmaf(p[k], bf_lo(vv[k].x), acc[0]);
+      acc[1] = fmaf(p[k], bf_hi(vv[k].x), acc[1]);
+      acc[2] = fmaf(p[k], bf_lo(vv[k].y), acc[2]);
+      acc[3] = fmaf(p[k], bf_hi(vv[k].y), acc[3]);
+    }
+    m = m_new;
+  }
+  uint16_t* orow = out + ((size_t)b * L + i) * QH * kAD + h * kAD + 4 * lane;
+  const float inv = 1.0f / l;
+  *reinterpret_cast<uint2*>(orow) = make_uint2(pack_bf2(acc[0] * inv, acc[1] * inv),
+                                               pack_bf2(acc[2] * inv, acc[3] * inv));
+}
+
 }  // namespace
 
 extern "C" {
@@ -803,6 +1351,111 @@ int q35_gqa_decode_fused(const void* packed, const void* q_w, const void* k_w, i
   if (e) return e;
   launch_combine(acc, ml, (const uint16_t*)packed, (uint16_t*)out, QH, splits,
                  (long long*)cache_len_dev, stream);
+  return q35_last_error();
+}
+
+// Split plan of the 64-key-block prefill kernel: query tile t (16 rows) has
+// nblk(t) key blocks and splits them into ranges of sb blocks, one workgroup
+// each. sb starts at 4 and grows until the workgroups of a prompt that starts
+// at key 0 fit one round on the device's CUs (one workgroup per CU: the
+// kernel takes 156 KB of LDS); smax = the splits of a tile covering the whole
+// cache sizes the grid and the workspace. The plan depends only on
+// (B, KVH, L, cache_len), so q35_gqa_prefill_workspace sees the same one.
+constexpr int kFaSplitBlocks = 4;
+static int fa_device_cus() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+      cus = n;
+    else
+      cus = 256;
+  }
+  return cus;
+}
+static void fa_plan(int B, int KVH, int L, int cache_len, int* sb_out, int* smax_out) {
+  const int nblk_max = (cache_len + kFaKeys - 1) / kFaKeys;
+  const int ntiles = (L + 15) / 16;
+  const long long budget = fa_device_cus();
+  int sb = kFaSplitBlocks;
+  for (; sb < nblk_max; ++sb) {
+    long long wgs = 0;
+    for (int t = 0; t < ntiles; ++t) {
+      const int nb = (min(16 * t + 16, L) + kFaKeys - 1) / kFaKeys;
+      wgs += (nb + sb - 1) / sb;
+    }
+    if (wgs * B * KVH <= budget) break;
+  }
+  *sb_out = sb;
+  *smax_out = (nblk_max + sb - 1) / sb;
+}
+
+long long q35_gqa_prefill_workspace(int B, int QH, int KVH, int L, int cache_len) {
+  if (B <= 0 || KVH <= 0 || QH <= 0 || QH % KVH || L <= 0 || cache_len <= 0) return 0;
+  const int G = QH / KVH;
+  if (G != 2 && G != 4) return 0;
+  int sb, smax;
+  fa_plan(B, KVH, L, cache_len, &sb, &smax);
+  if (smax <= 1) return 0;
+  return (long long)B * KVH * ((L + 15) / 16) * smax * G * 16 * (kAD + 2);
+}
+
+int q35_gqa_prefill(const void* q, const void* K, const void* V, void* out, int B, int QH, int KVH,
+                    int D, int L, int cache_len, int kv_start, const void* valid_len, float scale,
+                    void* workspace, long long workspace_floats, hipStream_t stream) {
+  Q35_CHECK_ARG(D == kAD && KVH > 0 && QH % KVH == 0 && B >= 0 && L >= 0);
+  Q35_CHECK_ARG(L <= cache_len && (valid_len || (kv_start >= 0 && kv_start + L <= cache_len)));
+  Q35_CHECK_ARG(q35_aligned16(q) && q35_aligned16(K) && q35_aligned16(V) && q35_aligned16(out));
+  if ((long long)B * QH * L == 0) return 0;
+  const int G = QH / KVH;
+  if ((G == 1 || G == 2 || G == 4 || G == 8) && B < 65536 && KVH < 65536) {
+    dim3 grid((unsigned)((L + 15) / 16), (unsigned)KVH, (unsigned)B);
+#define Q35_PF(GG)                                                                                  \
+  gqa_prefill_mfma<GG><<<grid, GG * 64, 0, stream>>>((const uint16_t*)q, (const uint16_t*)K,       \
+                                                     (const uint16_t*)V, (uint16_t*)out, B, QH, KVH, \
+                                                     L, cache_len, kv_start,                       \
+                                                     (const long long*)valid_len, scale)
+    if (G == 2 || G == 4) {
+      // Long query tiles split their key range over workgroups of at most
+      // kFaSplitBlocks blocks when the workspace holds the split records.
+      const int ntiles = (L + 15) / 16;
+      int sb, smax;
+      fa_plan(B, KVH, L, cache_len, &sb, &smax);
+      const long long need = q35_gqa_prefill_workspace(B, QH, KVH, L, cache_len);
+      if (smax <= 1 || !workspace || workspace_floats < need) {
+        smax = 1;
+        sb = (cache_len + kFaKeys - 1) / kFaKeys;
+      }
+      Q35_CHECK_ARG((long long)ntiles * smax < (1ll << 31));
+      dim3 fgrid((unsigned)(ntiles * smax), (unsigned)KVH, (unsigned)B);
+#define Q35_FA(GG)                                                                               \
+  do {                                                                                         \
+    gqa_prefill_fa<GG><<<fgrid, 2 * GG * 64, 0, stream>>>(                                     \
+        (const uint16_t*)q, (const uint16_t*)K, (const uint16_t*)V, (uint16_t*)out, B, QH, KVH,  \
+        L, cache_len, kv_start, (const long long*)valid_len, scale, sb, smax,                    \
+        (float*)workspace);                                                                      \
+    if (smax > 1)                                                                              \
+      gqa_prefill_merge<GG><<<grid, GG * 256, 0, stream>>>(                                    \
+          (const float*)workspace, (uint16_t*)out, B, QH, KVH, L, cache_len, kv_start,           \
+          (const long long*)valid_len, sb, smax);                                                \
+  } while (0)
+      if (G == 2) Q35_FA(2);
+      else Q35_FA(4);
+#undef Q35_FA
+    } else if (G == 1) {
+      Q35_PF(1);
+    } else {
+      Q35_PF(8);
+    }
+#undef Q35_PF
+    return q35_last_error();
+  }
+  const long long waves = (long long)B * QH * L;
+  Q35_CHECK_ARG(waves < (1ll << 31));
+  gqa_prefill_rows<<<(unsigned)((waves + 3) / 4), 256, 0, stream>>>(
+      (const uint16_t*)q, (const uint16_t*)K, (const uint16_t*)V, (uint16_t*)out, B, QH, KVH, L,
+      cache_len, kv_start, (const long long*)valid_len, scale);
   return q35_last_error();
 }
 
