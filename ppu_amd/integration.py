@@ -36,6 +36,8 @@ from typing import Any, Callable
 import torch
 from torch.autograd import forward_ad
 from torch.nn.modules import module as module_hooks
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 from transformers.activations import GELUTanh
 from transformers.cache_utils import DynamicCache
 from transformers.models.qwen3_5 import modeling_qwen3_5 as qwen_impl
@@ -86,10 +88,15 @@ def _gpu_bf16(t: Any) -> bool:
 def _values_only(*tensors: torch.Tensor) -> bool:
     """Whether a product of these tensors may be taken from their memory alone:
     no gradient, forward-mode tangent, autocast or function transform (vmap and
-    its like, whose tensors have no storage) asks for more, and no compiler is
-    tracing the call."""
-    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or forward_ad._current_level >= 0
-                or any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
+    its like, whose tensors have no storage) asks for more, and no tracer,
+    compiler or dispatch / function mode (a default device aside) has to see
+    the call."""
+    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or forward_ad._current_level >= 0
+                or torch._C._len_torch_dispatch_stack() or torch._ops._len_torch_dispatch_stack_pre_dispatch()
+                or (torch._C._len_torch_function_stack()
+                    and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
+                or torch._C._functorch.peek_interpreter_stack() is not None
                 or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
 
 
@@ -266,10 +273,10 @@ def _lm_head_fast(module):
     GEMV in 222. Further rows, biases and gradients stay with the module."""
     def fast(x, *args, **kwargs):
         w = module.weight
-        if (args or kwargs or not isinstance(x, torch.Tensor) or x.dim() == 0 or x.numel() != x.shape[-1]
-                or module.bias is not None or not (_gpu_bf16(x) and _gpu_bf16(w)) or x.device != w.device
-                or x.shape[-1] != w.shape[1] or not w.is_contiguous()
-                or not _values_only(x, w) or (x.data_ptr() | w.data_ptr()) % 16):
+        if (args or kwargs or module.bias is not None or not (_gpu_bf16(x) and _gpu_bf16(w))
+                or not _values_only(x, w) or x.device != w.device
+                or x.dim() == 0 or x.numel() != x.shape[-1] or x.shape[-1] != w.shape[1]
+                or not w.is_contiguous() or (x.data_ptr() | w.data_ptr()) % 16):
             return NotImplemented
         return K.linear(x, w)
     return fast
@@ -699,9 +706,10 @@ def _bias_linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, gelu:
     weights) 7.7 / 12.5 for proj, 19.4 / 22.2 fc2, 12 / 15 qkv, 15 / 17.6 fc1
     with its GELU; the tower 2615 / 2853, and its host time per uncaptured
     call is 15 % less."""
-    if (b is not None and x.dim() == 2 and x.shape[0] and _gpu_bf16(x) and _gpu_bf16(w) and _gpu_bf16(b)
-            and w.device == x.device == b.device and w.shape[1] == x.shape[1] and w.shape[1] % 64 == 0
-            and w.is_contiguous() and b.is_contiguous() and _values_only(x, w, b) and w.data_ptr() % 16 == 0
+    if (b is not None and _gpu_bf16(x) and _gpu_bf16(w) and _gpu_bf16(b) and _values_only(x, w, b)
+            and w.device == x.device == b.device and x.dim() == 2 and x.shape[0]
+            and w.shape[1] == x.shape[1] and w.shape[1] % 64 == 0
+            and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
             and max(x.shape[0], w.shape[0]) * w.shape[1] < 1 << 30):
         x = x.contiguous()
         if x.data_ptr() % 16 == 0:

@@ -3,9 +3,16 @@ values only, and modules whose hooks nobody would miss."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.autograd import forward_ad
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import _disable_current_modes
+from torch.utils.flop_counter import FlopCounterMode
 
 from ppu_amd import integration
 
@@ -45,3 +52,63 @@ def test_global_hook_sees_the_linear():
     finally:
         handle.remove()
     assert calls == [1]
+
+
+@pytest.fixture
+def head(monkeypatch):
+    """A language model head on the CPU whose fast path is taken as on the GPU
+    and, as there, writes its output through its address alone."""
+    def by_address(x, w):
+        y = torch.empty(*x.shape[:-1], w.shape[0], dtype=x.dtype)
+        with _disable_current_modes():
+            value = torch.nn.functional.linear(x.detach().clone(), w.detach().clone())
+        ctypes.memmove(y.data_ptr(), value.data_ptr(), value.numel() * value.element_size())
+        return y
+
+    linear = torch.nn.Linear(8, 4, bias=False).to(torch.bfloat16).requires_grad_(False)
+    monkeypatch.setattr(integration, "_gpu_bf16", lambda t: t.dtype == torch.bfloat16)
+    monkeypatch.setattr(integration.K, "linear", by_address)
+    integration._take_over(linear, integration._lm_head_fast(linear))
+    return linear
+
+
+def _row(seed):
+    return torch.randn(1, 8, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16)
+
+
+def test_plain_call_takes_the_fast_path(head, monkeypatch):
+    taken = []
+    monkeypatch.setattr(integration.K, "linear", lambda x, w: taken.append(1) or x[:, :4])
+    with torch.device("cpu"):  # a default device is not a tracer
+        head(_row(1))
+    assert taken == [1]
+
+
+@pytest.mark.parametrize("trace", [
+    lambda f, x: torch.jit.trace(f, x, check_trace=False), lambda f, x: make_fx(f)(x),
+    lambda f, x: make_fx(f, pre_dispatch=True)(x)])
+def test_traced_head_computes_its_logits(head, trace):
+    traced = trace(lambda x: head(x), _row(1))
+    x = _row(2)
+    assert torch.equal(traced(x), torch.nn.functional.linear(x, head.weight))
+
+
+def test_modes_see_the_product(head):
+    with FlopCounterMode(display=False) as flops:
+        head(_row(1))
+    assert flops.get_total_flops() == 2 * 8 * 4
+    with FakeTensorMode() as mode:
+        x, w = mode.from_tensor(_row(1)), mode.from_tensor(head.weight)
+        assert not integration._values_only(x, w) and not integration._values_only(x)
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        assert not integration._values_only(_row(1))
+    seen = []
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        head(_row(1))
+    assert torch.nn.functional.linear in seen or torch._C._nn.linear in seen
