@@ -85,18 +85,23 @@ def _gpu_bf16(t: Any) -> bool:
     return isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.bfloat16
 
 
+_DENSE = (torch.Tensor, torch.nn.Parameter)
+
+
 def _values_only(*tensors: torch.Tensor) -> bool:
     """Whether a product of these tensors may be taken from their memory alone:
     no gradient, forward-mode tangent, autocast or function transform (vmap and
-    its like, whose tensors have no storage) asks for more, and no tracer,
-    compiler or dispatch / function mode (a default device aside) has to see
-    the call."""
+    its like, whose tensors have no storage) asks for more, no tracer, compiler
+    or dispatch / function mode (a default device aside) has to see the call,
+    and they are dense tensors of torch's own classes: a subclass (quantised,
+    distributed, fake) or a sparse or nested one keeps its own product."""
     return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing()
                 or forward_ad._current_level >= 0
                 or torch._C._len_torch_dispatch_stack() or torch._ops._len_torch_dispatch_stack_pre_dispatch()
                 or (torch._C._len_torch_function_stack()
                     and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
                 or torch._C._functorch.peek_interpreter_stack() is not None
+                or any(type(t) not in _DENSE or t.layout is not torch.strided or t.is_nested for t in tensors)
                 or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)))
 
 

@@ -112,3 +112,44 @@ def test_modes_see_the_product(head):
     with Mode():
         head(_row(1))
     assert torch.nn.functional.linear in seen or torch._C._nn.linear in seen
+
+
+class _Packed(torch.Tensor):
+    """A wrapper subclass as quantised weights are: it says cuda and bf16, has
+    no storage and multiplies in its own way."""
+
+    @staticmethod
+    def __new__(cls, shape):
+        return torch.Tensor._make_wrapper_subclass(cls, shape, dtype=torch.bfloat16, device="cuda")
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        if func is torch.nn.functional.linear:
+            return "its own product"
+        with torch._C.DisableTorchFunctionSubclass():
+            return func(*args, **(kwargs or {}))
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        if func is torch.ops.aten.detach.default:
+            return _Packed(args[0].shape)
+        raise NotImplementedError(func)
+
+
+def test_weight_subclass_keeps_its_product(head):
+    head.weight = torch.nn.Parameter(_Packed((4, 8)), requires_grad=False)
+    assert head(_row(1)) == "its own product"
+    x, w, b = _row(1), torch.randn(4, 64).to(torch.bfloat16), torch.randn(4).to(torch.bfloat16)
+    assert integration._values_only(x, w, torch.nn.Parameter(b, requires_grad=False))
+    assert not integration._values_only(x, head.weight, b) and not integration._values_only(_Packed((1, 8)), w, b)
+    assert integration._bias_linear(x, head.weight, b) == "its own product"
+
+
+def test_sparse_and_nested_operands_keep_the_module(head):
+    rows = [_row(1).float(), _row(2).float()]
+    with torch.no_grad():
+        assert not integration._values_only(torch.nested.nested_tensor(rows))
+        dense = head.weight.float()
+        assert not integration._values_only(dense.to_sparse_csr()) and not integration._values_only(dense.to_sparse())
+        nested = torch.nested.nested_tensor([r.to(torch.bfloat16) for r in rows])
+        assert head(nested).is_nested
