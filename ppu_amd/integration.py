@@ -23,7 +23,8 @@ How it is put together here:
   combine + gate in another, the post-attention norm in the SwiGLU GEMV).
 
 Fields added for MI355X: ``fused_decode`` (use ``decode_layer`` for batch-1
-single-token steps over a static cache) and ``a8w8`` (the packed projections
+single-token steps over a static cache, and the decode GEMV for the lm_head's
+logits of one position) and ``a8w8`` (the packed projections
 and the other linears as A8W8, as reference explore_runtime_quantization.py
 applies PPUA8W8Linear; the lm_head stays bf16).
 """
@@ -1078,7 +1079,8 @@ def install(model: torch.nn.Module, config: FusionConfig,
     if config.vision and visual is not None:
         stats["vision"] = install_vision(visual, config)
     lm_head = getattr(model, "lm_head", None)
-    if type(lm_head) is torch.nn.Linear and lm_head.in_features == 2048:
+    # (other widths would run too; 2048 is the one measured)
+    if config.fused_decode and type(lm_head) is torch.nn.Linear and lm_head.in_features == 2048:
         _take_over(lm_head, _lm_head_fast(lm_head))
     model._qwen35_fusion_config = config
     stats["lm_head_screen"] = int(config.lm_head_screen and attach_lm_head_screen(model))

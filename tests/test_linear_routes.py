@@ -153,3 +153,16 @@ def test_sparse_and_nested_operands_keep_the_module(head):
         assert not integration._values_only(dense.to_sparse_csr()) and not integration._values_only(dense.to_sparse())
         nested = torch.nested.nested_tensor([r.to(torch.bfloat16) for r in rows])
         assert head(nested).is_nested
+
+
+def test_head_is_taken_over_with_fused_decode_only():
+    """Every fusion off leaves the head as it was."""
+    off = dict.fromkeys(("delta", "rms_norm", "residual_norm", "swiglu", "attention", "vision", "lm_head_screen"),
+                        False)
+    for fused in (False, True):
+        model = torch.nn.Module()
+        model.model = torch.nn.Module()
+        model.model.layers = torch.nn.ModuleList()
+        model.lm_head = torch.nn.Linear(2048, 4, bias=False)
+        integration.install(model.eval(), integration.FusionConfig(**off, fused_decode=fused), [])
+        assert ("forward" in model.lm_head.__dict__) == fused
