@@ -281,7 +281,7 @@ def _lm_head_fast(module):
         w = module.weight
         if (args or kwargs or module.bias is not None or not (_gpu_bf16(x) and _gpu_bf16(w))
                 or not _values_only(x, w) or x.device != w.device
-                or x.dim() == 0 or x.numel() != x.shape[-1] or x.shape[-1] != w.shape[1]
+                or x.dim() == 0 or x.numel() != x.shape[-1] or x.shape[-1] != w.shape[1] or not w.numel()
                 or not w.is_contiguous() or (x.data_ptr() | w.data_ptr()) % 16):
             return NotImplemented
         return K.linear(x, w)
@@ -713,7 +713,7 @@ def _bias_linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, gelu:
     with its GELU; the tower 2615 / 2853, and its host time per uncaptured
     call is 15 % less."""
     if (b is not None and _gpu_bf16(x) and _gpu_bf16(w) and _gpu_bf16(b) and _values_only(x, w, b)
-            and w.device == x.device == b.device and x.dim() == 2 and x.shape[0]
+            and w.device == x.device == b.device and x.dim() == 2 and x.numel() and w.shape[0]
             and w.shape[1] == x.shape[1] and w.shape[1] % 64 == 0
             and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
             and max(x.shape[0], w.shape[0]) * w.shape[1] < 1 << 30):

@@ -166,3 +166,20 @@ def test_head_is_taken_over_with_fused_decode_only():
         model.lm_head = torch.nn.Linear(2048, 4, bias=False)
         integration.install(model.eval(), integration.FusionConfig(**off, fused_decode=fused), [])
         assert ("forward" in model.lm_head.__dict__) == fused
+
+
+@pytest.mark.parametrize("n,k", [(0, 64), (4, 0)])
+def test_empty_linear_keeps_the_library(monkeypatch, n, k):
+    """No columns or no terms: F.linear answers (nothing, the bias), the GEMM's
+    entry refuses."""
+    def refused(*args, **kwargs):
+        raise RuntimeError
+
+    monkeypatch.setattr(integration, "_gpu_bf16", lambda t: t.dtype == torch.bfloat16)
+    monkeypatch.setattr(integration.K, "gemm_bias", refused)
+    monkeypatch.setattr(integration.K, "linear", refused)
+    x, w, b = (torch.ones(*s, dtype=torch.bfloat16) for s in ((3, k), (n, k), (n,)))
+    assert torch.equal(integration._bias_linear(x, w, b), torch.ones(3, n, dtype=torch.bfloat16))
+    head = torch.nn.Linear(k, n, bias=False).to(torch.bfloat16).requires_grad_(False)
+    integration._take_over(head, integration._lm_head_fast(head))
+    assert head(x[:1]).shape == (1, n)
