@@ -715,7 +715,7 @@ def _bias_linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, gelu:
     if (b is not None and _gpu_bf16(x) and _gpu_bf16(w) and _gpu_bf16(b) and _values_only(x, w, b)
             and w.device == x.device == b.device and x.dim() == 2 and x.numel() and w.shape[0]
             and w.shape[1] == x.shape[1] and w.shape[1] % 64 == 0
-            and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
+            and b.shape == w.shape[:1] and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
             and max(x.shape[0], w.shape[0]) * w.shape[1] < 1 << 30):
         x = x.contiguous()
         if x.data_ptr() % 16 == 0:

@@ -170,8 +170,8 @@ def test_head_is_taken_over_with_fused_decode_only():
 
 @pytest.mark.parametrize("n,k", [(0, 64), (4, 0)])
 def test_empty_linear_keeps_the_library(monkeypatch, n, k):
-    """No columns or no terms: F.linear answers (nothing, the bias), the GEMM's
-    entry refuses."""
+    """No columns or no terms, or one bias for all columns: F.linear answers,
+    the GEMM's entry refuses."""
     def refused(*args, **kwargs):
         raise RuntimeError
 
@@ -180,6 +180,8 @@ def test_empty_linear_keeps_the_library(monkeypatch, n, k):
     monkeypatch.setattr(integration.K, "linear", refused)
     x, w, b = (torch.ones(*s, dtype=torch.bfloat16) for s in ((3, k), (n, k), (n,)))
     assert torch.equal(integration._bias_linear(x, w, b), torch.ones(3, n, dtype=torch.bfloat16))
+    one = torch.ones(1, dtype=torch.bfloat16)  # a bias for every column
+    assert integration._bias_linear(torch.ones(3, 64, dtype=torch.bfloat16), w.new_ones(4, 64), one).eq(65).all()
     head = torch.nn.Linear(k, n, bias=False).to(torch.bfloat16).requires_grad_(False)
     integration._take_over(head, integration._lm_head_fast(head))
     assert head(x[:1]).shape == (1, n)
