@@ -708,15 +708,18 @@ def _text_fast(stack, config: FusionConfig):
 def _bias_linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, gelu: bool = False) -> torch.Tensor:
     """A vision linear (``gelu``: with the tanh GELU on its output): the
     hand-written GEMM where its operand rules hold and no gradient or autocast
-    is asked for, else the library's. At 784 patches the two take (us, cold
-    weights) 7.7 / 12.5 for proj, 19.4 / 22.2 fc2, 12 / 15 qkv, 15 / 17.6 fc1
-    with its GELU; the tower 2615 / 2853, and its host time per uncaptured
-    call is 15 % less."""
+    is asked for, up to 6.5e9 multiply-adds, else the library's. Timed with
+    cold weights over the tower's seven products at 16 to 9216 patches, the
+    library takes 1.02 to 1.7 times as long below that line (one exception,
+    0.98 for qkv at 1156-1225) and 0.76 to 1.2 times above it: at 784 patches
+    16.1 / 12.3 us for proj, 28.8 / 25.8 fc2, 19.5 / 18.3 qkv, 22.8 / 20.0 fc1
+    with its GELU, at 1800 29.7 / 39.0 for fc1, 45.0 / 49.0 fc2."""
     if (b is not None and _gpu_bf16(x) and _gpu_bf16(w) and _gpu_bf16(b) and _values_only(x, w, b)
             and w.device == x.device == b.device and x.dim() == 2 and x.numel() and w.shape[0]
             and w.shape[1] == x.shape[1] and w.shape[1] % 64 == 0
             and b.shape == w.shape[:1] and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
-            and max(x.shape[0], w.shape[0]) * w.shape[1] < 1 << 30):
+            and max(x.shape[0], w.shape[0]) * w.shape[1] < 1 << 30
+            and x.shape[0] * w.numel() <= 6.5e9):
         x = x.contiguous()
         if x.data_ptr() % 16 == 0:
             return K.gemm_bias(x, w, b, gelu=gelu)

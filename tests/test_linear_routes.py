@@ -185,3 +185,17 @@ def test_empty_linear_keeps_the_library(monkeypatch, n, k):
     head = torch.nn.Linear(k, n, bias=False).to(torch.bfloat16).requires_grad_(False)
     integration._take_over(head, integration._lm_head_fast(head))
     assert head(x[:1]).shape == (1, n)
+
+
+@pytest.mark.parametrize("m,n,k,ours", [(784, 4352, 1152, True), (1296, 4352, 1152, True), (1444, 4352, 1152, False),
+                                        (1800, 1152, 4352, False), (4096, 1152, 1152, True),
+                                        (306, 4608, 4608, True), (400, 4608, 4608, False)])
+def test_linear_route_by_work(monkeypatch, m, n, k, ours):
+    """The hand-written product where it is the faster one, the library's from
+    6.5e9 multiply-adds up."""
+    taken = []
+    monkeypatch.setattr(integration, "_gpu_bf16", lambda t: t.dtype == torch.bfloat16)
+    monkeypatch.setattr(integration.K, "gemm_bias", lambda x, w, b, gelu: taken.append(True))
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w, b: taken.append(False))
+    integration._bias_linear(*(torch.empty(*s, dtype=torch.bfloat16) for s in ((m, k), (n, k), (n,))))
+    assert taken == [ours]
