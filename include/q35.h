@@ -412,6 +412,11 @@ int q35_gemm(const void* A, const void* B, void* C, int M, int N, int K, int kin
              const void* s_w, int tile, int splits, void* workspace, long long workspace_bytes,
              void* stream);
 
+/* The tile that q35_gemm's default plan takes for a shape (host only): 0-10 a
+ * ring tile, from 11 on a tile of the K-splitting kernel; kinds 5 and 6 are
+ * q35_gemm_bias without and with gelu. -1 for sizes that the entries refuse. */
+int q35_gemm_plan(int M, int N, int K, int kind);
+
 /* C[M, N] = bf16(A . B^T + bias) (A [M, K], B [N, K], bias [N], all bf16), or
  * with gelu the tanh-approximated GELU of the sum, both on the fp32
  * accumulators: F.linear with a bias, and fc1 -> GELU, of the vision tower

@@ -85,6 +85,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "q35_dequant_i32": (_I, [_P, _P, _P, _P, _I, _I, _P]),
     "q35_dequant_swiglu_i32": (_I, [_P, _P, _P, _P, _I, _I, _P]),
     "q35_gemm_workspace": (_L, [_I, _I, _I, _I, _I, _I]),
+    "q35_gemm_plan": (_I, [_I, _I, _I, _I]),
     "q35_gemm": (_I, [_P, _P, _P, _I, _I, _I, _I, _P, _P, _I, _I, _P, _L, _P]),
     "q35_gemm_bias": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "q35_residual_rmsnorm_dequant_quant": (

@@ -824,6 +824,17 @@ long long q35_gemm_workspace(int M, int N, int K, int kind, int tile, int splits
   return workspace_bytes(tile, M, N, kind, splits);
 }
 
+// Tile of the default plan (host only): 0-10 the ring kernel's, from 11 on the
+// K-splitting kernel's, for the kinds of q35_gemm and 5 / 6 = q35_gemm_bias
+// without / with gelu; -1 for sizes that the entries refuse.
+int q35_gemm_plan(int M, int N, int K, int kind) {
+  if (M <= 0 || N <= 0 || K <= 0 || kind < 0 || kind > KIND_BIAS_GELU) return -1;
+  if (((long long)K * (kind_i8(kind) ? 1 : 2)) % kRB) return -1;
+  int tile = -1, splits = 1;
+  plan(M, N, K, kind, &tile, &splits);
+  return tile;
+}
+
 // Prefill GEMM C = A . B^T of the given kind (0 bf16, 1 bf16 SwiGLU, 2 int8 ->
 // int32, 3 int8 -> bf16 dequant, 4 int8 SwiGLU; see gemm.hip's header).
 // K * element bytes a multiple of 128 (the stage width); A and B 16-byte
