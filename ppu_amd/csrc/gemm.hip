@@ -707,6 +707,11 @@ void plan(int M, int N, int K, int kind, int* tile, int* splits) {
     // 4 and 7 are tiles 0 and 6 with another ring or walk: never faster
     if (t == 4 || t == 7 || (direct ? t == 0 || t == 1 || t == 9 : !kStaged[t])) continue;
     if (kind_swiglu(kind) && (t == 1 || t == 2)) continue;  // few columns per tile: the epilogue outweighs
+    // 256x256 from 16 stages: the fit above does not hold for its prologue and
+    // epilogue alone (us, against the next best tile: 441x9456 bf16 K = 128
+    // 18.9 / 11.1, 1356x6784 K = 640 32.0 / 27.4, 554x15536 K = 768 35.1 / 31.9;
+    // from 16 stages on never behind: 1141x12832 K = 1024 41.3 / 47.3)
+    if (t >= 9 && nk < 16) continue;
     const double us = ring_us(t, M, N, nk, kind);
     if (*tile < 0 || us < best) {
       best = us;

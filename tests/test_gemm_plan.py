@@ -6,6 +6,8 @@ from __future__ import annotations
 
 import pytest
 
+import pytest
+
 from ppu_amd import _lib
 
 
@@ -14,3 +16,17 @@ def test_refused_sizes():
     assert plan(0, 8, 64, 0) == plan(8, 0, 64, 0) == plan(8, 8, 0, 0) == -1
     assert plan(8, 8, 96, 0) == plan(8, 8, 64, 2) == plan(8, 8, 64, 7) == plan(8, 8, 64, -1) == -1
     assert plan(8, 8, 64, 0) >= 0 and plan(8, 8, 128, 2) >= 0
+
+
+@pytest.mark.parametrize("kind,m,n", [(0, 441, 9456), (2, 441, 9456), (1, 4780, 4888), (4, 1299, 7664), (0, 8838, 5128)])
+def test_widest_tile_from_16_stages(kind, m, n):
+    """256x256 needs 16 stages of 128 bytes to pay for its prologue and epilogue."""
+    plan = _lib.load().q35_gemm_plan
+    stage = 128 if kind in (2, 3, 4) else 64
+    assert all(plan(m, n, stage * nk, kind) not in (9, 10) for nk in range(1, 16))
+
+
+def test_widest_tile_for_whole_rounds():
+    plan = _lib.load().q35_gemm_plan
+    assert plan(8192, 2048, 6144, 0) == 10 and plan(4000, 4090, 1024, 0) == 10
+    assert plan(4000, 4090, 2048, 1) == 9 and plan(8192, 2048, 6144, 3) == 9

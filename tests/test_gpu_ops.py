@@ -1330,9 +1330,10 @@ def test_gemm_bf16_rejects_k():
         K.gemm_bf16(torch.zeros(4, 96, dtype=BF), torch.zeros(8, 96, dtype=BF))
 
 
-# (m, n, k) whose default plan is the 256x256 ring tile (whole rounds of it),
-# ragged in tokens and columns
-@pytest.mark.parametrize("m,n,k", [(4000, 4090, 256), (8100, 2048, 192)])
+# (m, n, k) whose default plan is the 256x256 ring tile (whole rounds of it, 16
+# stages or more; the int8 kinds at K = 2048 only), ragged in tokens and
+# columns, and two of fewer stages, whose plan is another tile
+@pytest.mark.parametrize("m,n,k", [(4000, 4090, 256), (8100, 2048, 192), (4000, 4090, 2048), (8100, 2048, 1024)])
 def test_gemm_256_tile(gpu, m, n, k):
     """The widest ring tile, chosen by the default plan only: bf16 (direct) and
     SwiGLU (staged) against fp64, int8 kinds bit-exact."""
