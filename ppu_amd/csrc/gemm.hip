@@ -682,7 +682,8 @@ double ring_us(int tile, int M, int N, int nk, int kind) {
 // 1024 (192 rows) 14.8 / 13.8; 2048x6144 bf16 M = 33 10.1 / 31.4, 340 23.5 /
 // 33.9, 600 30.2 / 35.0; int8 with the dequant M = 33 6.7 / 25.0, 340 13.4 /
 // 25.0, 1024 (192 rows) 22.2 / 24.9, to int32 at 512 15.1 / 19.0, at 1024 20.2 /
-// 20.1; 5120x2048 M = 256 13.8 / 15.9, 340 (192 rows) 16.0 / 15.4; 8320x2048 M =
+// 20.1; 5120x2048 M = 256 13.8 / 15.9, 340 (192 rows) 16.0 / 15.4,
+// to int32 (160 rows) 14.6 / 14.2; 8320x2048 M =
 // 96 16.4 / 17.1, 128 (192 rows) 18.6 / 17.5; 12288x2048 SwiGLU bf16 M = 64 14.9 /
 // 25.5, 128 19.6 / 29.1, 230 (256 rows) 25.5 / 26.9, int8 180 (224 rows) 15.9 /
 // 16.7, 230 (256 rows) 18.4 / 16.9.
@@ -690,7 +691,8 @@ void plan(int M, int N, int K, int kind, int* tile, int* splits) {
   const int es = kind_i8(kind) ? 1 : 2;
   const bool direct = kind_direct(kind);
   *splits = 1;
-  const int rows = kind == KIND_SWIGLU ? 256 : kind == KIND_DEQ_SWIGLU ? 224 : kind == KIND_DEQ && N <= 4096 ? 192 : 160;
+  const int rows = kind == KIND_SWIGLU ? 256 : kind == KIND_DEQ_SWIGLU ? 224 : kind == KIND_DEQ && N <= 4096 ? 192
+                 : kind == KIND_I32 && N > 4096 ? 128 : 160;
   for (int c = 0; c < kKsTiles; ++c) {
     if (kKsWeights[c] + kKsTokens[c] > rows) break;
     if (kind_swiglu(kind) ? !kKsSwiglu[c] : !kKsPlain[c]) continue;

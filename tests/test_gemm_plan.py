@@ -30,3 +30,12 @@ def test_widest_tile_for_whole_rounds():
     plan = _lib.load().q35_gemm_plan
     assert plan(8192, 2048, 6144, 0) == 10 and plan(4000, 4090, 1024, 0) == 10
     assert plan(4000, 4090, 2048, 1) == 9 and plan(8192, 2048, 6144, 3) == 9
+
+
+@pytest.mark.parametrize("m", [200, 256])
+def test_int32_of_wide_outputs_leaves_the_ksplit_kernel(m):
+    """Outputs wider than 4096 take the K-splitting kernel up to 128 operand rows
+    only (64 x 96 tiles were slower than one round of the ring's)."""
+    plan = _lib.load().q35_gemm_plan
+    assert plan(m, 5120, 2048, 2) < 11 and plan(160, 5120, 2048, 2) >= 11
+    assert plan(m, 2048, 2048, 2) >= 11 and plan(m, 5120, 2048, 0) >= 11
