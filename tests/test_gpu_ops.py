@@ -17,6 +17,7 @@ import torch
 from oracle import a8w8 as oa
 from oracle import ops as ref
 from tests.conftest import KERNEL_SEED, gen
+from tests.test_gemm_plan import cases as plan_cases
 
 pytestmark = pytest.mark.gpu
 
@@ -1330,10 +1331,9 @@ def test_gemm_bf16_rejects_k():
         K.gemm_bf16(torch.zeros(4, 96, dtype=BF), torch.zeros(8, 96, dtype=BF))
 
 
-# (m, n, k) whose default plan is the 256x256 ring tile (whole rounds of it, 16
-# stages or more; the int8 kinds at K = 2048 only), ragged in tokens and
-# columns, and two of fewer stages, whose plan is another tile
-@pytest.mark.parametrize("m,n,k", [(4000, 4090, 256), (8100, 2048, 192), (4000, 4090, 2048), (8100, 2048, 1024)])
+# (m, n, k) whose default plan is the 256x256 ring tile (whole rounds of it),
+# ragged in tokens and columns
+@pytest.mark.parametrize("m,n,k", [(4000, 4090, 256), (8100, 2048, 192)])
 def test_gemm_256_tile(gpu, m, n, k):
     """The widest ring tile, chosen by the default plan only: bf16 (direct) and
     SwiGLU (staged) against fp64, int8 kinds bit-exact."""
@@ -1465,6 +1465,65 @@ def test_gemm_ksplit_int8_exact(gpu, m, n, k):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y2, y)
+
+
+@pytest.mark.parametrize("kind,tile,m,n,k", [(kind, *c) for kind in range(7) for c in plan_cases(kind)])
+def test_gemm_default_tiles(gpu, kind, tile, m, n, k):
+    """Every tile of the default plan in every kind, ragged, against fp64 of the
+    same operands: int32 and dequantised values bit-exact, the others within
+    the fp32 sum of their terms and their bf16 roundings; no write past the
+    output, the same bits on a second launch."""
+    from ppu_amd import kernels as K, _lib
+
+    assert _lib.load().q35_gemm_plan(m, n, k, kind) == tile
+    g = torch.Generator(device=gpu).manual_seed(KERNEL_SEED + 101)
+    swiglu, int8 = kind in (1, 4), kind in (2, 3, 4)
+    rows = 2 * n if swiglu else n
+    x = torch.randn(m, k, device=gpu, generator=g).to(BF)
+    w = (torch.randn(rows, k, device=gpu, generator=g) * 2 * k**-0.5).to(BF)
+    out = torch.full((m + 1, n), 7, dtype=torch.int32 if kind == 2 else BF, device=gpu)
+    y = out[:m]
+    if int8:
+        wq, sw = K.quantize_weight_i8(w)
+        xq, sx = K.quantize_act_i8(x)
+        sw, sx = sw.reshape(-1), sx.reshape(-1)
+        launch = lambda c: K.gemm_into(xq, wq, c, kind, s_x=sx, s_w=sw)
+        acc = xq.double() @ wq.double().t()  # exact: |sum| < 2^53
+        deq = (acc.float() * sx.view(-1, 1) * sw.view(1, -1)).to(BF)
+        launch(y)
+        if not swiglu:
+            assert torch.equal(y, acc.to(torch.int32) if kind == 2 else deq)
+        ref, err = deq.double(), torch.zeros_like(acc)
+    else:
+        b = torch.randn(n, device=gpu, generator=g).to(BF) * 2
+        if kind < 2:
+            launch = lambda c: K.gemm_into(x, w, c, kind)
+        else:
+            launch = lambda c: _lib.call("q35_gemm_bias", x.data_ptr(), w.data_ptr(), b.data_ptr(), c.data_ptr(), m, n,
+                                         k, kind - 5, _lib.stream(x.device))
+        launch(y)
+        ref = x.double() @ w.double().t()
+        err = (k + 1) * 2.0**-24 * (x.double().abs() @ w.double().abs().t())  # the fp32 sum of k terms (and a bias)
+        if swiglu:
+            err = err + 2.0**-8 * ref.abs()  # bf16 of gate and up: half an ulp of 8 significand bits
+        elif kind > 4:
+            ref, err = ref + b.double(), err + (k + 1) * 2.0**-24 * b.double().abs()
+            if kind == 6:
+                # GELU's slope is at most 1.13; its exponential and reciprocal are right to 2^-15
+                ref = torch.nn.functional.gelu(ref, approximate="tanh")
+                err = 1.13 * err + 2.0**-15 * ref.abs()
+    if swiglu:
+        # |silu'| <= 1.1; silu's exponential and reciprocal are right to 2^-15, then it is rounded to bf16
+        (gate, up), (eg, eu) = (ref[:, :n], ref[:, n:]), (err[:, :n], err[:, n:])
+        silu = torch.nn.functional.silu(gate)
+        es = 1.1 * eg + (2.0**-8 + 2.0**-15) * (silu.abs() + 1.1 * eg)
+        ref, err = silu * up, es * (up.abs() + eu) + silu.abs() * eu
+    if swiglu or not int8:
+        assert bool(((y.double() - ref).abs() <= err + 2.0**-8 * (ref.abs() + err) + 1e-30).all())
+    assert bool((out[m] == 7).all())
+    again = torch.empty_like(y)
+    launch(again)
+    assert torch.equal(again, y)
 
 
 @pytest.mark.parametrize("m", [3, 8, 16])
