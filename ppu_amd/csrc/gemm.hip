@@ -50,8 +50,8 @@
 // s_barrier, then the first fragments of stage kt + 1 are read under the
 // second half.
 //
-// Split K (for outputs with fewer tiles than CUs): `splits` workgroups per
-// tile each take kps stages. Each stores its partial tile (fp32 / int32 bit
+// Split K (a caller's plan, or the default one for the dequant kind at K of
+// 10240 and more): `splits` workgroups per tile each take kps stages. Each stores its partial tile (fp32 / int32 bit
 // patterns, in accumulator-register order so every wave store is 512
 // contiguous bytes) with agent-scope stores, every thread waits until its
 // stores have completed (s_waitcnt vmcnt(0)), and one thread counts the
@@ -654,7 +654,8 @@ long long workspace_bytes(int tile, int M, int N, int kind, int splits) {
 // Time of one workgroup of a ring tile with all CUs busy: kFixed + kStage per
 // stage of 128 bytes, in us (fits of outputs 2048 to 12288 wide with K = 2048
 // and 6144 bf16 or int8; by tile, 1 and 6, 0 and 5, 9 and 10 alike). kDequant:
-// what the dequant epilogue adds (9 also with SwiGLU, about half).
+// what the dequant epilogue adds (9 also with SwiGLU, about half; there it holds
+// all 512 registers and 8-16 bytes per lane in scratch memory).
 constexpr double kFixed[kTiles] = {11.6, 5.7, 7, 7.7, 11.6, 11.6, 5.7, 5.7, 4.8, 5.1, 5.1};
 constexpr double kStage[kTiles] = {1.06, 0.51, 0.92, 0.667, 1.06, 1.06, 0.51, 0.51, 0.353, 1.7, 1.7};
 constexpr double kDequant[kTiles] = {0, 1.3, 2, 0.5, 0, 0, 0, 0, 0, 10, 0};
@@ -671,13 +672,24 @@ double ring_us(int tile, int M, int N, int nk, int kind) {
   return one * (whole + (rest > 0 ? (whole < 3 ? 0.7 + 0.3 * rest : 0.45 + 0.5 * rest) : 0));
 }
 
+// Operand rows (weights + tokens) up to which an output takes the K-splitting
+// kernel; the figures stand at plan().
+constexpr int ks_rows(int kind, int N) {
+  return kind == KIND_SWIGLU ? 256 : kind == KIND_DEQ_SWIGLU ? 224 : kind == KIND_DEQ && N <= 4096 ? 192
+         : kind == KIND_I32 && N > 4096 ? 128 : 160;
+}
+
 // Default plan. Large outputs: the ring tile with the least estimated time,
-// direct stores for the bf16 / int32 kinds and the staged epilogue for SwiGLU
-// and dequant. What it decides is the last round of CUs: the down projection
-// (2048x6144) at 4096 tokens has 176 tiles of 256x192 (116 us) but 256 of
-// 256x128 (95 us), at 2003 tokens 66 us on 256x192 and 54 us on 128x128. Outputs
-// with fewer 128x128 tiles than CUs split K only when each split keeps at least
-// 40 stages (the partial-tile exchange costs more than the idle CUs below that).
+// direct stores for the bf16 / int32 kinds (tiles 2 and 3 are built staged only)
+// and the staged epilogue for SwiGLU and dequant. What it decides is the last
+// round of CUs: the down projection (2048x6144) at 4096 tokens has 176 tiles of
+// 256x192 (116 us) but 256 of 256x128 (95 us), at 2003 tokens 66 us on 256x192 and
+// 54 us on 128x128. The estimates hold from K = 2048 bytes up or so; over 238
+// random shapes of 1 to 15 stages nine took 6-9 % longer than on the tile that
+// the tile counts alone suggest. 128x128 tiles on at most half the CUs split K
+// only when each split keeps at least 40 stages (the partial-tile exchange costs
+// more than the idle CUs below that); that leaves the dequant kind, where no
+// 128x64 tile takes such outputs.
 //
 // Outputs of few tokens or few columns run on the K-splitting kernel instead
 // (tile kTiles + its index): the smallest of its tiles that covers the output
@@ -687,17 +699,16 @@ double ring_us(int tile, int M, int N, int nk, int kind) {
 // 1024 (192 rows) 14.8 / 13.8; 2048x6144 bf16 M = 33 10.1 / 31.4, 340 23.5 /
 // 33.9, 600 30.2 / 35.0; int8 with the dequant M = 33 6.7 / 25.0, 340 13.4 /
 // 25.0, 1024 (192 rows) 22.2 / 24.9, to int32 at 512 15.1 / 19.0, at 1024 20.2 /
-// 20.1; 5120x2048 M = 256 13.8 / 15.9, 340 (192 rows) 16.0 / 15.4,
-// to int32 (160 rows) 14.6 / 14.2; 8320x2048 M =
-// 96 16.4 / 17.1, 128 (192 rows) 18.6 / 17.5; 12288x2048 SwiGLU bf16 M = 64 14.9 /
-// 25.5, 128 19.6 / 29.1, 230 (256 rows) 25.5 / 26.9, int8 180 (224 rows) 15.9 /
-// 16.7, 230 (256 rows) 18.4 / 16.9.
+// 20.1; 5120x2048 M = 256 13.8 / 15.9, 340 (192 rows) 16.0 / 15.4, to int32 (160
+// rows) 14.6 / 14.2; 8320x2048 M = 96 16.4 / 17.1, 128 (192 rows) 18.6 / 17.5;
+// 12288x2048 SwiGLU bf16 M = 64 14.9 / 25.5, 128 19.6 / 29.1, 230 (256 rows) 25.5 /
+// 26.9, int8 180 (224 rows) 15.9 / 16.7, 230 (256 rows) 18.4 / 16.9. The row
+// limits lie between the sides that these figures show.
 void plan(int M, int N, int K, int kind, int* tile, int* splits) {
   const int es = kind_i8(kind) ? 1 : 2;
   const bool direct = kind_direct(kind);
   *splits = 1;
-  const int rows = kind == KIND_SWIGLU ? 256 : kind == KIND_DEQ_SWIGLU ? 224 : kind == KIND_DEQ && N <= 4096 ? 192
-                 : kind == KIND_I32 && N > 4096 ? 128 : 160;
+  const int rows = ks_rows(kind, N);
   for (int c = 0; c < kKsTiles; ++c) {
     if (kKsWeights[c] + kKsTokens[c] > rows) break;
     if (kind_swiglu(kind) ? !kKsSwiglu[c] : !kKsPlain[c]) continue;
@@ -735,9 +746,6 @@ void plan(int M, int N, int K, int kind, int* tile, int* splits) {
 
 template <int WM, int WN, int FM, int FN, int RB, int NSA, int NSB, bool ROT, int KIND, bool STAGED>
 int launch_one(const GemmArgs& a, hipStream_t stream) {
-  if constexpr (!STAGED && !kind_direct(KIND)) {
-    return (int)hipErrorInvalidValue;  // direct stores: bf16 and int32 kinds
-  } else {
   constexpr int TM = WM * FM * 32, TN = WN * FN * 32;
   constexpr int NC = kind_swiglu(KIND) ? TN / 2 : TN;
   const long long units = (long long)((a.M + TM - 1) / TM) * ((a.N + NC - 1) / NC) * a.splits;
@@ -752,36 +760,37 @@ int launch_one(const GemmArgs& a, hipStream_t stream) {
     gemm_ring<WM, WN, FM, FN, RB, NSA, NSB, ROT, KIND, false, STAGED><<<(unsigned)units, 256, 0, stream>>>(a);
   }
   return q35_last_error();
-  }
 }
 
-template <int FN, int FM, int W, int S, bool HALF, bool SWIGLU, bool PLAIN, int KIND>
-int launch_ks(const GemmArgs& a, hipStream_t stream) {
-  if constexpr (kind_swiglu(KIND) ? SWIGLU : PLAIN) return launch_ksplit<FN, FM, W, S, HALF, KIND>(a, stream);
-  else return (int)hipErrorInvalidValue;
+// Tiles that a kind can run on (the others are not built): what the default
+// plan takes, and for the kinds of q35_gemm the ring tiles 0-8 of a caller's plan.
+constexpr bool has_tile(int kind, int tile) {
+  if (tile >= kTiles) {
+    const int c = tile - kTiles;
+    return (kind_swiglu(kind) ? kKsSwiglu[c] : kKsPlain[c]) && kKsWeights[c] + kKsTokens[c] <= ks_rows(kind, 1);
+  }
+  if (kind_bias(kind)) return tile != 0 && tile != 1 && tile != 4 && tile != 7 && tile != 9;
+  return kind_direct(kind) ? tile != 9 : kStaged[tile];
 }
 
 template <int KIND>
 int launch_tile(int tile, const GemmArgs& a, hipStream_t stream) {
-  if constexpr (kind_bias(KIND)) {
-    // q35_gemm_bias has the default plan only: the tiles it takes for the direct
-    // kinds, unsplit
-    switch (tile) {
-      case 0: case 1: case 4: case 7: case 9: return (int)hipErrorInvalidValue;
-      default: break;
-    }
-  }
   switch (tile) {
 #define Q35_GEMM_KS_CASE(id, fn, fm, w, s, half, sg, pl) \
-  case kTiles + id: return launch_ks<fn, fm, w, s, half, sg, pl, KIND>(a, stream);
+  case kTiles + id: \
+    if constexpr (has_tile(KIND, kTiles + id)) return launch_ksplit<fn, fm, w, s, half, KIND>(a, stream); \
+    break;
     Q35_GEMM_KS_TILES(Q35_GEMM_KS_CASE)
 #undef Q35_GEMM_KS_CASE
 #define Q35_GEMM_CASE(id, wm, wn, fm, fn, rb, nsa, nsb, rot, staged) \
-  case id: return launch_one<wm, wn, fm, fn, rb, nsa, nsb, rot, KIND, staged>(a, stream);
+  case id: \
+    if constexpr (has_tile(KIND, id)) return launch_one<wm, wn, fm, fn, rb, nsa, nsb, rot, KIND, staged>(a, stream); \
+    break;
     Q35_GEMM_TILES(Q35_GEMM_CASE)
 #undef Q35_GEMM_CASE
-    default: return (int)hipErrorInvalidValue;
+    default: break;
   }
+  return (int)hipErrorInvalidValue;
 }
 
 int gemm_run(const void* A, const void* B, void* C, int M, int N, int K, int kind, const float* s_x,

@@ -75,6 +75,7 @@ __global__ __launch_bounds__(W * 64) void gemm_ksplit(const GemmArgs a) {
   constexpr int HV = FN * FM > 8 ? 2 : 1;  // a piece's fragments in registers at once, or half of them
   using AccT = typename GemmAcc<I8>::T;
   using QuadT = typename GemmAcc<I8>::Q;
+  static_assert(S <= 3, "the waits count one or S - 1 pieces in flight");
   static_assert(!HALF || (FN == 1 && !SWIGLU), "a half tile is one block whose rows 16..31 repeat 0..15");
   static_assert(!SWIGLU || FN % 2 == 0, "SwiGLU tiles hold gate and up rows");
   // the sum: partial blocks (32 x 32, 4 KiB) of every wave, as many at a time as fit
@@ -149,7 +150,6 @@ __global__ __launch_bounds__(W * 64) void gemm_ksplit(const GemmArgs a) {
   for (int t = 0; t < nw; ++t) {
     // this piece landed: at most the copies of the pieces after it are left
     if (S > 1 && t + S <= nw) wait_vm<(S - 1) * NG>();
-    else if (S > 2 && t + 2 < nw) wait_vm<(S > 2 ? 2 : 0) * NG>();
     else if (S > 1 && t + 1 < nw) wait_vm<(S > 1 ? 1 : 0) * NG>();
     else wait_vm<0>();
     asm volatile("" ::: "memory");

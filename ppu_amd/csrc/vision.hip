@@ -755,7 +755,7 @@ int q35_vision_attention(const void* q, const void* k, const void* v, void* out,
                                                                           n_images, tokens, heads, dim, scale)
   // 128 keys per stage (8 waves, one workgroup per CU by LDS) while the grid
   // leaves CUs idle; 64 (4 waves, two workgroups per CU) for larger grids and
-  // for the 128-dim tiles, whose registers do not fit two waves per SIMD.
+  // for head dims over 96, which already take all 256 registers in that form.
   const bool split = grid < 512;
 #define VA_PICK(KT_)      \
   if (split)              \

@@ -1331,7 +1331,8 @@ def test_gemm_bf16_rejects_k():
         K.gemm_bf16(torch.zeros(4, 96, dtype=BF), torch.zeros(8, 96, dtype=BF))
 
 
-# (m, n, k) whose default plan is the 256x256 ring tile (whole rounds of it),
+# (m, n, k) of whole rounds of the 256x256 ring tile (the plan takes it from 16
+# stages of K on; test_gemm_default_tiles has one each),
 # ragged in tokens and columns
 @pytest.mark.parametrize("m,n,k", [(4000, 4090, 256), (8100, 2048, 192)])
 def test_gemm_256_tile(gpu, m, n, k):
