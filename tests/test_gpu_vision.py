@@ -180,8 +180,8 @@ def _rel(a, b):
 
 
 def test_vision_tower_matches_transformers_and_graph_replays(gpu):
-    """The fused vision forward (our LayerNorm / position-embedding / RoPE
-    kernels, library GEMMs, the vision_attn_fa flash kernel) against Transformers' fp32 CPU forward
+    """The fused vision forward (LayerNorm / position-embedding / RoPE kernels,
+    the GEMM with bias and GELU, the vision_attn_fa flash kernel) against Transformers' fp32 CPU forward
     of the same weights; the second call of a patch count replays the captured
     graph and every replay (with eager work in between) equals the eager call."""
     from qwen35_fused.integration import apply_fusions
@@ -267,6 +267,74 @@ def test_vision_attention_per_image(gpu, bounds, heads):
     for a, b in zip(bounds[:-1], bounds[1:]):
         if b - a == 1:
             assert torch.equal(got[a].cpu().reshape(heads, dim), v[0, :, a])
+
+
+# every count of head-dim steps (8 to 128 in 16s, odd multiples of 8 too), both
+# stage forms (grids below and from 512 workgroups), tile and stage edges; the
+# key lengths grow along the tokens, so the row maxima keep moving
+@pytest.mark.parametrize("tokens,heads,dim", [(130, 2, 16), (65, 3, 24), (300, 2, 32), (129, 1, 40), (383, 2, 48),
+                                              (257, 2, 56), (511, 1, 64), (640, 2, 88), (321, 2, 96), (200, 2, 104),
+                                              (449, 1, 112), (127, 2, 120), (900, 40, 72), (833, 48, 40), (1500, 24, 80)])
+def test_vision_attention_moving_maxima(gpu, tokens, heads, dim):
+    """fp64 attention of the same operands; P is rounded to bf16 (2^-8 of each
+    term), the result once more, scores and sums carry the fp32 error."""
+    from ppu_amd import kernels as K
+
+    g = gen(KERNEL_SEED + 8)
+    q, k, v = (randn(g, 1, heads, tokens, dim) for _ in range(3))
+    k = (k * torch.linspace(0.5, 5.0, tokens).view(-1, 1)).to(k.dtype)
+    got = K.vision_attention(q.to(gpu), k.to(gpu), v.to(gpu), dim ** -0.5).double()
+    qd, kd, vd = (t[0].to(gpu).double() for t in (q, k, v))
+    for h in range(heads):
+        p = torch.softmax(qd[h] @ kd[h].t() * dim ** -0.5, dim=-1)
+        # relative error of p: that of its score, |score| up to 100, and the base-2 exponential
+        scores = (qd[h].abs() @ kd[h].abs().t()).amax() * dim ** -0.5
+        rel = 2.0**-8 + 2 * (dim + 2) * 2.0**-24 * float(scores) + 2.0**-20
+        exp, mass = p @ vd[h], p @ vd[h].abs()
+        bound = 2 * rel * mass + 2.0**-8 * exp.abs() + 1e-30  # numerator and denominator
+        assert bool(((got[:, h * dim : (h + 1) * dim] - exp).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("bounds,heads", [([0, 128, 257], 2), ([0, 128, 1153], 32), ([0, 100, 257], 2), ([0, 37, 64], 2)])
+def test_vision_attention_other_images_values(gpu, bounds, heads):
+    """NaN and infinities in another image: its keys never reach a row, its
+    values not from another tile of 64 rows."""
+    from ppu_amd import kernels as K
+
+    g = gen(KERNEL_SEED + 9)
+    dim, tokens, cut = 72, bounds[-1], bounds[1]
+    q, k, v = (randn(g, 1, heads, tokens, dim).to(gpu) for _ in range(3))
+    cu = torch.tensor(bounds, dtype=torch.int32, device=gpu)
+    clean = K.vision_attention(q, k, v, dim ** -0.5, cu)
+    for bad in (float("nan"), float("inf"), float("-inf")):
+        kb, vb = k.clone(), v.clone()
+        kb[:, :, cut:] = bad
+        if cut % 64 == 0:
+            vb[:, :, cut:] = bad
+        got = K.vision_attention(q, kb, vb, dim ** -0.5, cu)
+        assert torch.equal(got[:cut], clean[:cut])
+        kb, vb = k.clone(), v.clone()
+        kb[:, :, :cut] = bad
+        if cut % 64 == 0:
+            vb[:, :, :cut] = bad
+        got = K.vision_attention(q, kb, vb, dim ** -0.5, cu)
+        assert torch.equal(got[cut:], clean[cut:])
+
+
+@pytest.mark.parametrize("tokens,dim", [(100, 72), (64, 128)])
+def test_vision_attention_unaligned_output(gpu, tokens, dim):
+    """An output that starts at a 2-byte boundary (C entry only): the same
+    values, nothing written around it."""
+    from ppu_amd import _lib, kernels as K
+
+    g = gen(KERNEL_SEED + 10)
+    q, k, v = (randn(g, 1, 2, tokens, dim).to(gpu) for _ in range(3))
+    exp = K.vision_attention(q, k, v, dim ** -0.5)
+    buf = torch.full((exp.numel() + 8,), 7.0, dtype=exp.dtype, device=gpu)
+    _lib.call("q35_vision_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), buf[1:].data_ptr(), None, 0, tokens, 2,
+              dim, dim ** -0.5, _lib.stream(q.device))
+    assert torch.equal(buf[1 : 1 + exp.numel()].view_as(exp), exp)
+    assert bool((buf[:1] == 7).all()) and bool((buf[1 + exp.numel() :] == 7).all())
 
 
 def test_vision_mlp_fused_gelu_matches_module(gpu):
