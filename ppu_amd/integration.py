@@ -32,6 +32,7 @@ applies PPUA8W8Linear; the lm_head stays bf16).
 from __future__ import annotations
 
 from dataclasses import dataclass
+from types import MethodType
 from typing import Any, Callable
 
 import torch
@@ -286,6 +287,20 @@ def _lm_head_fast(module):
             return NotImplemented
         return K.linear(x, w)
     return fast
+
+
+def _take_over_head(module: torch.nn.Linear) -> None:
+    """``_take_over`` for the lm_head, through a bound method: a copy of the
+    head (deepcopy, pickle) is bound to its own weight."""
+    if getattr(module, "_q35_original_forward", None) is not None:
+        return
+
+    def forward(self, *args, **kwargs):
+        out = _lm_head_fast(self)(*args, **kwargs)
+        return self._q35_original_forward(*args, **kwargs) if out is NotImplemented else out
+
+    module._q35_original_forward = module.forward
+    module.forward = MethodType(forward, module)
 
 
 def _mlp_fast(module, config: FusionConfig):
@@ -1084,7 +1099,7 @@ def install(model: torch.nn.Module, config: FusionConfig,
     lm_head = getattr(model, "lm_head", None)
     # (other widths would run too; 2048 is the one measured)
     if config.fused_decode and type(lm_head) is torch.nn.Linear and lm_head.in_features == 2048:
-        _take_over(lm_head, _lm_head_fast(lm_head))
+        _take_over_head(lm_head)
     model._qwen35_fusion_config = config
     stats["lm_head_screen"] = int(config.lm_head_screen and attach_lm_head_screen(model))
     stats["delta_precompute_factors"] = int(config.delta and config.delta_precompute_factors)

@@ -3,7 +3,9 @@ values only, and modules whose hooks nobody would miss."""
 
 from __future__ import annotations
 
+import copy
 import ctypes
+import pickle
 
 import pytest
 import torch
@@ -155,17 +157,32 @@ def test_sparse_and_nested_operands_keep_the_module(head):
         assert head(nested).is_nested
 
 
-def test_head_is_taken_over_with_fused_decode_only():
-    """Every fusion off leaves the head as it was."""
+def _installed_head(fused):
     off = dict.fromkeys(("delta", "rms_norm", "residual_norm", "swiglu", "attention", "vision", "lm_head_screen"),
                         False)
-    for fused in (False, True):
-        model = torch.nn.Module()
-        model.model = torch.nn.Module()
-        model.model.layers = torch.nn.ModuleList()
-        model.lm_head = torch.nn.Linear(2048, 4, bias=False)
-        integration.install(model.eval(), integration.FusionConfig(**off, fused_decode=fused), [])
-        assert ("forward" in model.lm_head.__dict__) == fused
+    model = torch.nn.Module()
+    model.model = torch.nn.Module()
+    model.model.layers = torch.nn.ModuleList()
+    model.lm_head = torch.nn.Linear(2048, 4, bias=False)
+    integration.install(model.eval(), integration.FusionConfig(**off, fused_decode=fused), [])
+    return model.lm_head
+
+
+def test_head_is_taken_over_with_fused_decode_only():
+    """Every fusion off leaves the head as it was."""
+    assert "forward" in _installed_head(True).__dict__
+    assert "forward" not in _installed_head(False).__dict__
+
+
+@pytest.mark.parametrize("twin", [copy.deepcopy, lambda head: pickle.loads(pickle.dumps(head))])
+def test_copied_head_uses_its_own_weight(twin):
+    head = _installed_head(True)
+    other, x = twin(head), torch.ones(1, 2048)
+    with torch.no_grad():
+        other.weight.fill_(2.0)
+        assert other(x).eq(4096).all() and not head(x).eq(4096).any()
+    other(x).sum().backward()
+    assert other.weight.grad is not None and head.weight.grad is None
 
 
 @pytest.mark.parametrize("n,k", [(0, 64), (4, 0)])
