@@ -77,10 +77,10 @@
 // eighth of the units. M runs fastest within bands of 8 M tiles, so the 32
 // units that an XCD works on at a time are 8 M tiles x 4 N tiles and share both
 // operands (with all M tiles fastest, each XCD of 2048x6144 at 8192 tokens
-// streamed all 100 MB of activations for one N tile). In one round of
+// streamed all 100 MB of activations for one N tile). Short of a whole round of
 // CUs few M tiles are better off in one band (us, one band against bands of 8:
 // 2048x6144 bf16 10 M tiles 64.8 / 65.6, 20 82.0 / 85.0, but 23 153.9 / 149.5, 32
-// 166.9 / 160.1).
+// 166.9 / 160.1, and 16 with all 256 units 126.6 / 126.3).
 #include "gemm_ksplit.hpp"
 
 namespace {
@@ -153,9 +153,9 @@ __global__ __launch_bounds__(256, 1) void gemm_ring(const GemmArgs a) {
   const int U = ntiles * S;
   const int xcd = (int)blockIdx.x & 7;
   int u = xcd * (U >> 3) + min(xcd, U & 7) + ((int)blockIdx.x >> 3);
-  // bands of kBand M tiles (the last one smaller; up to 20 M tiles in one round
+  // bands of kBand M tiles (the last one smaller; up to 20 M tiles, with CUs to spare,
   // are one band): M tile fastest inside one
-  const int kb = U <= 256 && mt <= 20 ? mt : kBand;
+  const int kb = U <= 224 && mt <= 20 ? mt : kBand;
   const int band = u / (kb * nt * S);
   u -= band * (kb * nt * S);
   const int bm = min(kb, mt - band * kb);
