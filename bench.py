@@ -583,6 +583,11 @@ DECODE_ALGO_BYTES = {
 RESCORE_NAME = "lm_head_rescore<4>"
 
 
+def _own_gemm(name: str) -> bool:
+    """A launch of the hand-written matrix-core GEMMs (both kernels)."""
+    return "gemm_ring<" in name or "gemm_ksplit<" in name
+
+
 def trace_summary(kind: str, trace_csv: str, bench_json: str) -> None:
     """Print the per-kernel anatomy of a ``rocprofv3 --kernel-trace`` run of
     ``bench.py --no-cpu --no-kernels``: ``decode`` = one graph-replayed decode
@@ -605,11 +610,11 @@ def trace_summary(kind: str, trace_csv: str, bench_json: str) -> None:
         return (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
 
     def int8(a, b):
-        # int8 GEMV (last template argument true) or an int8 kind (>= 2) of
-        # the prefill GEMM (seventh template argument)
+        # int8 GEMV (last template argument true) or an int8 kind (2-4) of the
+        # prefill GEMM kernels
         def is_i8(name):
-            m = re.search(r"gemm_ring<(?:\s*\d+,){7}\s*\w+,\s*(\d+),", name)
-            return ("gemv_fused" in name and ", true>" in name) or (m is not None and int(m.group(1)) >= 2)
+            m = re.search(r"gemm_(?:ring<(?:\s*\d+,){7}\s*\w+|ksplit<(?:\s*\d+,){4}\s*\w+),\s*(\d+)[,>]", name)
+            return ("gemv_fused" in name and ", true>" in name) or (m is not None and 2 <= int(m.group(1)) <= 4)
         return any(is_i8(rows[i]["Kernel_Name"]) for i in range(a, b))
 
     def table(seg, grid, top=None):
@@ -638,7 +643,8 @@ def trace_summary(kind: str, trace_csv: str, bench_json: str) -> None:
         # before its position-embedding add; the last call ends the trace of
         # `bench.py --vision-only`
         starts = [i for i, r in enumerate(rows) if "position_embed_add_rows" in r["Kernel_Name"]]
-        gemms = [i for i, r in enumerate(rows) if r["Kernel_Name"].startswith("Cijk")]
+        gemms = [i for i, r in enumerate(rows)
+                 if r["Kernel_Name"].startswith("Cijk") or _own_gemm(r["Kernel_Name"])]
         if starts and gemms:
             # ... and ends with the merger's second GEMM and the two output copies
             a, b = max(starts[-1] - 1, 0), gemms[-1] + 1
@@ -762,13 +768,13 @@ def mfma_summary(pmc_csv: str, trace_csv: str) -> None:
     names = {}
     with open(pmc_csv) as f:
         for row in csv.DictReader(f):
-            if "gemm_ring" in row["Kernel_Name"]:
+            if _own_gemm(row["Kernel_Name"]):
                 d = int(row["Dispatch_Id"])
                 per[d][row["Counter_Name"]] = float(row["Counter_Value"])
                 names[d] = short(row["Kernel_Name"])
     cnt = [(names[d], per[d]) for d in sorted(per)]
     with open(trace_csv) as f:
-        rows = [r for r in csv.DictReader(f) if "gemm_ring" in r["Kernel_Name"]]
+        rows = [r for r in csv.DictReader(f) if _own_gemm(r["Kernel_Name"])]
     rows.sort(key=lambda r: int(r["Dispatch_Id"]))
     dur = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3 for r in rows]
     labels = [f"{n}x{k}{' SwiGLU' if sw else ''} {kind}" for n, k, sw in PROBE_GEMMS
