@@ -1331,13 +1331,13 @@ def test_gemm_bf16_rejects_k():
         K.gemm_bf16(torch.zeros(4, 96, dtype=BF), torch.zeros(8, 96, dtype=BF))
 
 
-# (m, n, k) of whole rounds of the 256x256 ring tile (the plan takes it from 16
-# stages of K on; test_gemm_default_tiles has one each),
-# ragged in tokens and columns
+# (m, n, k) of whole rounds of the 256x256 ring tile, ragged in tokens and
+# columns, with too few stages of K for it
 @pytest.mark.parametrize("m,n,k", [(4000, 4090, 256), (8100, 2048, 192)])
 def test_gemm_256_tile(gpu, m, n, k):
-    """The widest ring tile, chosen by the default plan only: bf16 (direct) and
-    SwiGLU (staged) against fp64, int8 kinds bit-exact."""
+    """Large outputs of short K on the default plan: bf16 (direct) and SwiGLU
+    (staged) against fp64, int8 kinds bit-exact. (The 256x256 tile itself:
+    test_gemm_default_tiles.)"""
     from ppu_amd import kernels as K
 
     g = gen(KERNEL_SEED + 96)
@@ -1358,9 +1358,9 @@ def test_gemm_256_tile(gpu, m, n, k):
         assert torch.equal(K.gemm_a8w8(xq, sx, wq, sw), deq)
 
 
-# (m, n, k) with the default plan on each tile of the K-splitting GEMM (few
-# tokens or columns), ragged in tokens and columns, one to many 128-byte pieces
-# of K per wave, and fewer pieces than waves
+# (m, n, k) of few tokens or columns, ragged, one to many 128-byte pieces of K per
+# wave and fewer pieces than waves: the K-splitting GEMM's tiles 0, 1, 2, 4, 6 (8
+# with the dequant) and one ring tile (every tile: test_gemm_default_tiles)
 _KS_SHAPES = [(2, 2048, 2048), (17, 2048, 6144), (65, 2045, 512), (100, 500, 1152), (33, 5120, 2048),
               (97, 5116, 256), (129, 2048, 640), (150, 5120, 128), (200, 2000, 6144), (340, 2048, 384),
               (500, 2044, 1024), (256, 5100, 2048), (784, 2048, 256), (1000, 1152, 512), (95, 8320, 2048)]
@@ -1387,7 +1387,7 @@ def test_gemm_ksplit_bf16(gpu, m, n, k):
     assert torch.equal(K.gemm_into(xd, wd, y2, K.GEMM_BF16), y[:m])
 
 
-# ring tiles (128x128 and 128-row direct, 256 wide) besides the K-splitting ones
+# K-splitting tiles 0, 4 and 6, ring tiles 2, 5 and 6 (every tile: test_gemm_default_tiles)
 @pytest.mark.parametrize("gelu", [False, True])
 @pytest.mark.parametrize("m,n,k", _KS_SHAPES[1:12:2] + [(784, 4352, 1152), (785, 3450, 320), (1600, 4304, 192),
                                                         (4100, 1154, 128), (4096, 4608, 256)])
